@@ -54,6 +54,27 @@ def test_attn_rope_equals_rope_then_attn(T, case):
     _rope_case(T, case)
 
 
+# prefill batches at the edges of the kernel's rotation table: rows and pairs
+# that do not fill it, a half-head that is no multiple of 8 elements (NEOX),
+# and one head per group, whose rows take two tables
+TABLE_CASES = [
+    (8, 8, 128, 3, 290, 128, 1, 5e5),
+    (8, 8, 64, 77, 257, 64, 0, 5e5),
+    (4, 4, 256, 50, 130, 256, 1, 1e4),
+    (14, 2, 128, 9, 33, 36, 1, 1e6),
+    (12, 4, 128, 40, 65, 20, 0, 1e4),
+    (8, 2, 256, 1, 31, 24, 1, 1e4),
+    (8, 1, 64, 500, 17, 2, 1, 1e4),
+]
+
+
+@pytest.mark.parametrize("case", TABLE_CASES)
+def test_attn_rope_prefill_table_edges(T, case):
+    import tlkv
+    with tlkv.tuning(tlkv.TUNE_NO_PREFILL, 2):
+        _rope_case(T, case)
+
+
 @pytest.mark.parametrize("case", [c for c in CASES if c[4] >= 16])
 def test_attn_rope_prefill_kernel_forced(T, case):
     """The batches of 16+ rows on the prefill kernel, also where the plan

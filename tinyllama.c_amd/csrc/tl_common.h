@@ -114,9 +114,11 @@ TL_DEV void rope_rot(float a, float b, float c, float s, float &x, float &y) {
     x = fmaf(a, c, -(b * s));
     y = fmaf(a, s, b * c);
 }
+TL_DEV float rope_theta(u32 i, u32 rdim, float base) {
+    return 1.0f / powf(base, (float)(2 * i) / (float)rdim);
+}
 TL_DEV void rope_cs(u32 i, u32 rdim, float base, u32 pos, float &c, float &s) {
-    const float th = 1.0f / powf(base, (float)(2 * i) / (float)rdim);
-    sincosf((float)pos * th, &s, &c);
+    sincosf((float)pos * rope_theta(i, rdim, base), &s, &c);
 }
 /* elements e0..e0+7 of one head row (hrow = its element 0), rotated at
  * position pos when rdim > 0 */
@@ -152,6 +154,64 @@ TL_DEV void load8_rope(const float *hrow, u32 e0, u32 pos, u32 rdim, float base,
             float c, s, x, y;
             rope_cs(i, rdim, base, pos, c, s);
             rope_rot(pa, pb, c, s, x, y);
+            out[j] = lo ? x : y;
+        }
+    }
+}
+
+/* The same rotation from a table of the row's (cos, sin) pairs: tab[i] holds
+ * rope_cs of pair i, formed with the same operations (rope_theta, then
+ * sincosf), so the bits are load8_rope's.  A kernel that rotates several heads
+ * of a row builds the table once per row instead of paying powf + sincosf per
+ * head and element. */
+TL_DEV void load8_rope_tab(const float *hrow, u32 e0, u32 rdim, int neox, const float2 *tab,
+                           float out[8]) {
+    const float4 a = *(const float4 *)(hrow + e0);
+    const float4 b = *(const float4 *)(hrow + e0 + 4);
+    out[0] = a.x; out[1] = a.y; out[2] = a.z; out[3] = a.w;
+    out[4] = b.x; out[5] = b.y; out[6] = b.z; out[7] = b.w;
+    if (e0 >= rdim) return;
+    if (!neox) {
+#pragma unroll
+        for (int j = 0; j < 8; j += 2) {
+            if (e0 + j < rdim) {
+                const float2 cs = tab[(e0 + j) >> 1];
+                float x, y;
+                rope_rot(out[j], out[j + 1], cs.x, cs.y, x, y);
+                out[j] = x;
+                out[j + 1] = y;
+            }
+        }
+        return;
+    }
+    const u32 half = rdim >> 1;
+    if ((half & 7) == 0) {
+        /* the 8 elements are all of the low or all of the high half */
+        const bool lo = e0 < half;
+        const u32 i0 = lo ? e0 : e0 - half;
+        const float *q = hrow + (lo ? e0 + half : i0);
+        const float4 c = *(const float4 *)q, d = *(const float4 *)(q + 4);
+        const float o[8] = {c.x, c.y, c.z, c.w, d.x, d.y, d.z, d.w};
+#pragma unroll
+        for (int j = 0; j < 8; j++) {
+            const float2 cs = tab[i0 + j];
+            float x, y;
+            rope_rot(lo ? out[j] : o[j], lo ? o[j] : out[j], cs.x, cs.y, x, y);
+            out[j] = lo ? x : y;
+        }
+        return;
+    }
+#pragma unroll
+    for (int j = 0; j < 8; j++) {
+        const u32 e = e0 + j;
+        if (e < rdim) {
+            const bool lo = e < half;
+            const u32 i = lo ? e : e - half;
+            const float pa = lo ? out[j] : hrow[i];
+            const float pb = lo ? hrow[e + half] : out[j];
+            const float2 cs = tab[i];
+            float x, y;
+            rope_rot(pa, pb, cs.x, cs.y, x, y);
             out[j] = lo ? x : y;
         }
     }
