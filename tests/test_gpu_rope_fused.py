@@ -54,10 +54,10 @@ def test_attn_rope_equals_rope_then_attn(T, case):
     _rope_case(T, case)
 
 
-# prefill batches at the edges of the kernel's rotation table: rows and pairs
-# that do not fill it, a half-head that is no multiple of 8 elements (NEOX),
-# and one head per group, whose rows take two tables
-TABLE_CASES = [
+# prefill batches at the edges of the rotating pre-launch: partial rotation,
+# a half-head that is no multiple of 8 elements (NEOX), heads that do and do
+# not fill its workgroups' passes
+PREP_CASES = [
     (8, 8, 128, 3, 290, 128, 1, 5e5),
     (8, 8, 64, 77, 257, 64, 0, 5e5),
     (4, 4, 256, 50, 130, 256, 1, 1e4),
@@ -65,14 +65,17 @@ TABLE_CASES = [
     (12, 4, 128, 40, 65, 20, 0, 1e4),
     (8, 2, 256, 1, 31, 24, 1, 1e4),
     (8, 1, 64, 500, 17, 2, 1, 1e4),
+    (64, 8, 256, 20, 18, 256, 1, 1e4),
 ]
 
 
-@pytest.mark.parametrize("case", TABLE_CASES)
-def test_attn_rope_prefill_table_edges(T, case):
+@pytest.mark.parametrize("in_place", [False, True])
+@pytest.mark.parametrize("case", PREP_CASES)
+def test_attn_rope_prefill_prep_edges(T, case, in_place):
+    """in_place: dst is q, which the pre-launch also uses for the rotated q."""
     import tlkv
     with tlkv.tuning(tlkv.TUNE_NO_PREFILL, 2):
-        _rope_case(T, case)
+        _rope_case(T, case, in_place)
 
 
 @pytest.mark.parametrize("case", [c for c in CASES if c[4] >= 16])
@@ -84,7 +87,7 @@ def test_attn_rope_prefill_kernel_forced(T, case):
         _rope_case(T, case)
 
 
-def _rope_case(T, case):
+def _rope_case(T, case, in_place=False):
     import tlkv
     n_head, n_kv, hd, pos, n, rdim, neox, theta = case
     lib = tlkv.lib()
@@ -111,12 +114,12 @@ def _rope_case(T, case):
     tlkv.check(lib.tl_attn(layers[0].desc, a1, None))
     # fused
     qs, ks = q0.clone(), k0.clone()
-    out2 = T.zeros((n, qd), dtype=T.float32, device="cuda")
+    out2 = q0 if in_place else T.zeros((n, qd), dtype=T.float32, device="cuda")
     a2 = tlkv.attn_args(q0, k0, v0, out2, slots, pos, n, n_head, hd, n_kv, 0, scale)
     rp = tlkv.RopeParams(rdim, theta, neox)
     tlkv.check(lib.tl_attn_rope(layers[1].desc, a2, rp, None))
     T.cuda.synchronize()
-    assert T.equal(q0, qs) and T.equal(k0, ks), "fused path modified its inputs"
+    assert (in_place or T.equal(q0, qs)) and T.equal(k0, ks), "fused path modified its inputs"
     assert np.array_equal(out1.cpu().numpy(), out2.cpu().numpy())
     g1 = _gather(T, tlkv, layers[0], slots, pos + n)
     g2 = _gather(T, tlkv, layers[1], slots, pos + n)

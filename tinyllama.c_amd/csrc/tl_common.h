@@ -161,15 +161,12 @@ TL_DEV void load8_rope(const float *hrow, u32 e0, u32 pos, u32 rdim, float base,
 
 /* The same rotation from a table of the row's (cos, sin) pairs: tab[i] holds
  * rope_cs of pair i, formed with the same operations (rope_theta, then
- * sincosf), so the bits are load8_rope's.  A kernel that rotates several heads
- * of a row builds the table once per row instead of paying powf + sincosf per
- * head and element. */
-TL_DEV void load8_rope_tab(const float *hrow, u32 e0, u32 rdim, int neox, const float2 *tab,
-                           float out[8]) {
-    const float4 a = *(const float4 *)(hrow + e0);
-    const float4 b = *(const float4 *)(hrow + e0 + 4);
-    out[0] = a.x; out[1] = a.y; out[2] = a.z; out[3] = a.w;
-    out[4] = b.x; out[5] = b.y; out[6] = b.z; out[7] = b.w;
+ * sincosf), so the bits are load8_rope's.  own: elements e0..e0+7; other:
+ * their partners for NEOX (rope_partner; unused for NORM). */
+TL_DEV bool rope_aligned8(u32 rdim, int neox) { return !neox || ((rdim >> 1) & 7) == 0; }
+TL_DEV u32 rope_partner(u32 e0, u32 rdim) { return e0 < rdim >> 1 ? e0 + (rdim >> 1) : e0 - (rdim >> 1); }
+TL_DEV void rope8_tab(float own[8], const float other[8], u32 e0, u32 rdim, int neox,
+                      const float2 *tab) {
     if (e0 >= rdim) return;
     if (!neox) {
 #pragma unroll
@@ -177,42 +174,38 @@ TL_DEV void load8_rope_tab(const float *hrow, u32 e0, u32 rdim, int neox, const 
             if (e0 + j < rdim) {
                 const float2 cs = tab[(e0 + j) >> 1];
                 float x, y;
-                rope_rot(out[j], out[j + 1], cs.x, cs.y, x, y);
-                out[j] = x;
-                out[j + 1] = y;
+                rope_rot(own[j], own[j + 1], cs.x, cs.y, x, y);
+                own[j] = x;
+                own[j + 1] = y;
             }
         }
         return;
     }
-    const u32 half = rdim >> 1;
-    if ((half & 7) == 0) {
-        /* the 8 elements are all of the low or all of the high half */
-        const bool lo = e0 < half;
-        const u32 i0 = lo ? e0 : e0 - half;
-        const float *q = hrow + (lo ? e0 + half : i0);
-        const float4 c = *(const float4 *)q, d = *(const float4 *)(q + 4);
-        const float o[8] = {c.x, c.y, c.z, c.w, d.x, d.y, d.z, d.w};
+    /* rope_aligned8: the 8 elements are all of the low or all of the high half */
+    const bool lo = e0 < rdim >> 1;
+    const u32 i0 = lo ? e0 : e0 - (rdim >> 1);
 #pragma unroll
-        for (int j = 0; j < 8; j++) {
-            const float2 cs = tab[i0 + j];
-            float x, y;
-            rope_rot(lo ? out[j] : o[j], lo ? o[j] : out[j], cs.x, cs.y, x, y);
-            out[j] = lo ? x : y;
-        }
-        return;
+    for (int j = 0; j < 8; j++) {
+        const float2 cs = tab[i0 + j];
+        float x, y;
+        rope_rot(lo ? own[j] : other[j], lo ? other[j] : own[j], cs.x, cs.y, x, y);
+        own[j] = lo ? x : y;
     }
+}
+/* any NEOX half: partners read from the row, element by element */
+TL_DEV void rope8_tab_any(float own[8], const float *hrow, u32 e0, u32 rdim, const float2 *tab) {
+    const u32 half = rdim >> 1;
 #pragma unroll
     for (int j = 0; j < 8; j++) {
         const u32 e = e0 + j;
         if (e < rdim) {
             const bool lo = e < half;
             const u32 i = lo ? e : e - half;
-            const float pa = lo ? out[j] : hrow[i];
-            const float pb = lo ? hrow[e + half] : out[j];
+            const float pr = hrow[lo ? e + half : i];
             const float2 cs = tab[i];
             float x, y;
-            rope_rot(pa, pb, cs.x, cs.y, x, y);
-            out[j] = lo ? x : y;
+            rope_rot(lo ? own[j] : pr, lo ? pr : own[j], cs.x, cs.y, x, y);
+            own[j] = lo ? x : y;
         }
     }
 }

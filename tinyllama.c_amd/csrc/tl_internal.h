@@ -98,14 +98,13 @@ struct PrefParams {
     const uint16_t *ks, *vs;  /* Q8_0 scales, else NULL */
     const uint32_t *slots;
     uint32_t cap, ring;
-    const float *q;
+    const float *q;           /* NULL: the rotated f16 q in dst (attn_rope_prep_kernel) */
     float *dst;
     uint32_t q_stride, pos, n, n_head, n_kv, window;
     float scale_log2;
     uint32_t n_split;
     float *ws_acc;
     float2 *ws_ml;
-    RopeCfg rope;            /* applied to q rows (and to appended K rows) */
     /* fused append (f16 cache; kin NULL: none): the batch's K/V rows, f32
      * [n][kv_stride], converted and written by the launch's own workgroups
      * in units of 16 rows of one kv-head; flags[kvh * units + u] = epoch once
@@ -114,6 +113,17 @@ struct PrefParams {
     const float *kin, *vin;
     uint32_t kv_stride, polls;
     uint32_t *flags, *ctr;
+};
+/* One rotating pre-launch of a prefill batch (attn_rope_prep_kernel). */
+struct PrepParams {
+    const float *q, *k, *v;
+    float *dst;
+    uint16_t *kc, *vc;        /* f16 rows, or int8 rows of a Q8_0 cache */
+    uint16_t *ks, *vs;        /* Q8_0 scales, else NULL */
+    const uint32_t *slots;
+    uint32_t cap, ring, pos, n, n_head, n_kv, q_stride, kv_stride;
+    float scale_log2;
+    RopeCfg rope;
 };
 /* the fused append's counters sit past the decode merge's in a workspace */
 #define TL_PF_CTR_WORDS 64
@@ -177,5 +187,7 @@ int tl_launch_merge(const DecParams &p, uint32_t n_rows_total, uint32_t head_dim
 bool tl_prefill_supported(const LayerView &L, const tl_attn_args *a);
 /* the batch runs on the prefill kernel (else on the decode kernel) */
 bool tl_use_prefill(const LayerView &L, const tl_attn_args *a);
+/* append: the launch writes the batch rows itself (f16 cache); with RoPE the
+ * rotating pre-launch writes them, into either cache */
 int tl_launch_prefill(const LayerView &L, const tl_attn_args *a, const RopeCfg &rope,
                       hipStream_t st, bool append = false);

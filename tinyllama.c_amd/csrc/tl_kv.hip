@@ -689,11 +689,12 @@ static int attn_core(const tl_kv_layer *L, const tl_attn_args *a, bool append,
             int rc = fill_seg(ap.seg[0], L, a->k, a->v, a->kv_stride, a->slots, a->pos, a->n);
             if (rc) return rc;
             /* the prefill launch writes the rows itself (its stores address
-             * the whole layer through one 2 GB buffer resource) */
+             * the whole layer through one 2 GB buffer resource); with RoPE
+             * its rotating pre-launch does */
+            if (rope.rdim) return tl_launch_prefill(lv, a, rope, st, true);
             fused = !tl_tune(TL_TUNE_PREFILL_SEPARATE_APPEND) &&
                     (u64)L->n_kv_head * L->cap * L->head_dim * 2 < 0x7ffffff0ull;
             if (!fused) {
-                ap.rope = rope;
                 rc = tl_launch_append(ap, 1, st);
                 if (rc) return rc;
             }

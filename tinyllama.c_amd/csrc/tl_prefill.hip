@@ -42,7 +42,151 @@
  */
 #include "tl_prefill_kernels.h"
 
-TL_PREFILL_PICKER(tl_prefill_fn, false, false)
+TL_PREFILL_PICKER(tl_prefill_fn, false)
+
+/* ------------------------------------------------------------------------ */
+/* RoPE of a prefill batch                                                   */
+/* ------------------------------------------------------------------------ */
+
+/* Before the attention launch of a batch with RoPE: q rotated, scaled to log2
+ * units and rounded to f16 as the kernel's MFMA operand, K rotated and
+ * appended, V appended (f16 or Q8_0: the append kernels' conversions).  One
+ * workgroup per row: a row's (cos, sin) pairs are formed once for all its
+ * heads, while the row's loads are in flight.  The f16 q goes where the
+ * attention output will be (the first half of each head's D floats of dst),
+ * so nothing is allocated; the attention launch reads it before that output
+ * is written.  The lanes of one head are of one wave and load before they
+ * store, so dst may be q.
+ *
+ * Bound by latency: one round trip for the row beside one sincosf, then the
+ * stores.  Rotated inside the attention launch instead, every key split and
+ * kv-head repeated the rotation before its first tile (us per OP_ATTN, with
+ * powf + sincosf per lane and element / with a table per workgroup / here):
+ * 333 rows from position 0 at 28/4/128 NEOX 77.9 / 28.6 / 23.7; 512 rows at
+ * 8/4/256 NEOX over a 1024-key window 131 / 49.0 / 37.1; 512 rows at 32/8/128
+ * over 4K keys of a Q8_0 cache (which always had an append launch) 84.7 /
+ * 67.0 / 62.6; 512 rows at 32/8/128 over 32K keys 312 / 290 / 294. */
+template <int D, bool Q8>
+__global__ __launch_bounds__(256) void attn_rope_prep_kernel(const PrepParams p) {
+    constexpr int VPR = D / 8, U = 4;
+    __shared__ float2 s_tab[D / 2];
+    const u32 tid = threadIdx.x, pairs = p.rope.rdim >> 1;
+    const u32 items = (p.n_head + 2 * p.n_kv) * VPR;
+    const bool part = p.rope.neox && rope_aligned8(p.rope.rdim, 1);
+    const float th = tid < pairs ? rope_theta(tid, p.rope.rdim, p.rope.theta) : 0.f;
+    for (u32 row = blockIdx.x; row < p.n; row += gridDim.x) {
+        const u32 key = p.pos + row;
+        const u32 ph = p.ring ? key % p.ring : (p.slots ? p.slots[key] : key);
+        for (u32 i0 = 0; i0 < items; i0 += 256 * U) {
+            /* item = 8 elements of one head: the q heads, then K, then V */
+            float x[U][8], y[U][8];
+            auto src_of = [&](u32 i) -> const float * {
+                const u32 hd = i / VPR;
+                if (hd < p.n_head) return p.q + (u64)row * p.q_stride + (u64)hd * D;
+                const bool kk = hd < p.n_head + p.n_kv;
+                return (kk ? p.k : p.v) + (u64)row * p.kv_stride +
+                       (u64)(hd - p.n_head - (kk ? 0u : p.n_kv)) * D;
+            };
+#pragma unroll
+            for (int u = 0; u < U; u++) {
+                const u32 i = i0 + u * 256 + tid, e0 = (i % VPR) * 8;
+                if (i < items) {
+                    const float *hrow = src_of(i);
+                    const float4 a = *(const float4 *)(hrow + e0), b = *(const float4 *)(hrow + e0 + 4);
+                    x[u][0] = a.x; x[u][1] = a.y; x[u][2] = a.z; x[u][3] = a.w;
+                    x[u][4] = b.x; x[u][5] = b.y; x[u][6] = b.z; x[u][7] = b.w;
+                    if (part && e0 < p.rope.rdim) {
+                        const u32 o = rope_partner(e0, p.rope.rdim);
+                        const float4 c = *(const float4 *)(hrow + o), d = *(const float4 *)(hrow + o + 4);
+                        y[u][0] = c.x; y[u][1] = c.y; y[u][2] = c.z; y[u][3] = c.w;
+                        y[u][4] = d.x; y[u][5] = d.y; y[u][6] = d.z; y[u][7] = d.w;
+                    }
+                }
+            }
+            if (i0 == 0) {
+                if (row != blockIdx.x) __syncthreads();   /* the previous row's readers */
+                if (tid < pairs) {
+                    float c, s;
+                    sincosf((float)key * th, &s, &c);
+                    s_tab[tid] = make_float2(c, s);
+                }
+                __syncthreads();
+            }
+#pragma unroll
+            for (int u = 0; u < U; u++) {
+                const u32 i = i0 + u * 256 + tid, e0 = (i % VPR) * 8, hd = i / VPR;
+                if (i >= items) continue;
+                if (hd < p.n_head + p.n_kv) {
+                    if (rope_aligned8(p.rope.rdim, p.rope.neox))
+                        rope8_tab(x[u], y[u], e0, p.rope.rdim, p.rope.neox, s_tab);
+                    else
+                        rope8_tab_any(x[u], src_of(i), e0, p.rope.rdim, s_tab);
+                }
+                if (hd < p.n_head) {
+                    const float sc = p.scale_log2;
+                    u16 *o = (u16 *)(p.dst + (u64)row * p.q_stride + (u64)hd * D) + e0;
+                    *(uint4 *)o = make_uint4(pack2(x[u][0] * sc, x[u][1] * sc), pack2(x[u][2] * sc, x[u][3] * sc),
+                                             pack2(x[u][4] * sc, x[u][5] * sc), pack2(x[u][6] * sc, x[u][7] * sc));
+                    continue;
+                }
+                const bool kk = hd < p.n_head + p.n_kv;
+                const u64 prow = (u64)(hd - p.n_head - (kk ? 0u : p.n_kv)) * p.cap + ph;
+                u16 *c = kk ? p.kc : p.vc;
+                if constexpr (Q8) {
+                    /* the 4 lanes of a 32-value block are an aligned group */
+                    const float d = group_max<4>(amax8(x[u])) / 127.0f;
+                    if (ph >= p.cap) continue;
+                    *(uint2 *)((uint8_t *)c + prow * D + e0) = q8_pack8(x[u], d > 0.0f ? 1.0f / d : 0.0f);
+                    if ((e0 & 31) == 0) (kk ? p.ks : p.vs)[prow * (D / 32) + e0 / 32] = (u16)f32_to_f16_bits(d);
+                } else {
+                    if (ph >= p.cap) continue;
+                    *(uint4 *)(c + prow * D + e0) =
+                        make_uint4(pack_f16x2(x[u][0], x[u][1]), pack_f16x2(x[u][2], x[u][3]),
+                                   pack_f16x2(x[u][4], x[u][5]), pack_f16x2(x[u][6], x[u][7]));
+                }
+            }
+        }
+    }
+}
+
+static const void *prep_fn(u32 D, bool q8) {
+    switch (D) {
+    case 64: return q8 ? (const void *)attn_rope_prep_kernel<64, true> : (const void *)attn_rope_prep_kernel<64, false>;
+    case 128: return q8 ? (const void *)attn_rope_prep_kernel<128, true> : (const void *)attn_rope_prep_kernel<128, false>;
+    case 256: return q8 ? (const void *)attn_rope_prep_kernel<256, true> : (const void *)attn_rope_prep_kernel<256, false>;
+    default: return nullptr;
+    }
+}
+
+static int launch_rope_prep(const LayerView &L, const tl_attn_args *a, const RopeCfg &rope, float scale_log2,
+                            hipStream_t st) {
+    PrepParams p;
+    memset(&p, 0, sizeof(p));
+    p.q = a->q;
+    p.k = a->k;
+    p.v = a->v;
+    p.dst = a->dst;
+    p.kc = (u16 *)L.k;
+    p.vc = (u16 *)L.v;
+    p.ks = (u16 *)L.ks;
+    p.vs = (u16 *)L.vs;
+    p.slots = a->slots;
+    p.cap = L.cap;
+    p.ring = L.ring;
+    p.pos = a->pos;
+    p.n = a->n;
+    p.n_head = a->n_head;
+    p.n_kv = L.n_kv_head;
+    p.q_stride = a->q_stride;
+    p.kv_stride = a->kv_stride;
+    p.scale_log2 = scale_log2;
+    p.rope = rope;
+    const void *fn = prep_fn(L.head_dim, L.q8);
+    if (!fn) return tl_fail(TL_EINVAL, "prefill: head_dim %u", L.head_dim);
+    void *args[] = {(void *)&p};
+    HIP_TRY(hipLaunchKernel(fn, dim3(a->n < 2048 ? a->n : 2048), dim3(256), args, 0, st));
+    return TL_OK;
+}
 
 /* ------------------------------------------------------------------------ */
 
@@ -79,7 +223,9 @@ static u32 qblocks(u32 D, u32 G) {
 
 int tl_launch_prefill(const LayerView &L, const tl_attn_args *a, const RopeCfg &rope,
                       hipStream_t st, bool append) {
-    if (append && L.q8) return tl_fail(TL_EINVAL, "prefill: no fused append into a Q8_0 cache");
+    const bool rope_on = rope.rdim != 0;
+    if (append && L.q8 && !rope_on)
+        return tl_fail(TL_EINVAL, "prefill: no fused append into a Q8_0 cache");
     const u32 D = L.head_dim, G = a->n_head / L.n_kv_head;
     if (L.q8 && (!L.ks || !L.vs)) return tl_fail(TL_EINVAL, "prefill: a Q8_0 cache needs scales");
     PrefParams p;
@@ -100,7 +246,11 @@ int tl_launch_prefill(const LayerView &L, const tl_attn_args *a, const RopeCfg &
     p.n_kv = L.n_kv_head;
     p.window = a->window;
     p.scale_log2 = a->scale * 1.4426950408889634f;
-    p.rope = rope;
+    if (rope_on) {
+        if (!append) return tl_fail(TL_EINVAL, "prefill: RoPE without the batch's K/V rows");
+        append = false;      /* the pre-launch below writes them */
+        p.q = nullptr;
+    }
 
     const u32 rows = 32 * qblocks(D, G);
     const u32 nqb = (a->n + rows - 1) / rows;
@@ -149,10 +299,12 @@ int tl_launch_prefill(const LayerView &L, const tl_attn_args *a, const RopeCfg &
         }
     }
     const u32 blocks = base * ns;
-    const bool rope_on = rope.rdim != 0;
-    const void *fn = L.q8 ? (rope_on ? tl_prefill_fn_q8_rope(D, G) : tl_prefill_fn_q8(D, G))
-                          : (rope_on ? tl_prefill_fn_rope(D, G) : tl_prefill_fn(D, G));
+    const void *fn = L.q8 ? tl_prefill_fn_q8(D, G) : tl_prefill_fn(D, G);
     if (!fn) return tl_fail(TL_EINVAL, "prefill: head_dim %u gqa %u", D, G);
+    if (rope_on) {
+        const int rc = launch_rope_prep(L, a, rope, p.scale_log2, st);
+        if (rc) return rc;
+    }
     void *args[] = {(void *)&p};
     HIP_TRY(hipLaunchKernel(fn, dim3(blocks), dim3(64 * G * qblocks(D, G)), args, 0, st));
     if (ns == 1) return TL_OK;

@@ -1,9 +1,7 @@
 /* tl_prefill_kernels.h — the chunked-prefill MFMA kernel (template) and its
  * device helpers, shared by the translation units that instantiate it:
- * tl_prefill.hip (f16 cache, launch code) and tl_prefill_rope.hip,
- * tl_prefill_q8.hip, tl_prefill_q8_rope.hip (one (RoPE, Q8_0) variant each,
- * so the instances build in parallel).  The design is described in
- * tl_prefill.hip. */
+ * tl_prefill.hip (f16 cache, launch code) and tl_prefill_q8.hip (Q8_0 cache).
+ * The design is described in tl_prefill.hip. */
 #pragma once
 #include "tl_common.h"
 #include "tl_internal.h"
@@ -53,7 +51,7 @@ TL_DEV uint2 ld_tr16(const _Float16 *lds_ptr) {
     return make_uint2(lo, hi);
 }
 
-template <int D, int G, bool ROPE, bool Q8>
+template <int D, int G, bool Q8>
 __global__ __attribute__((amdgpu_flat_work_group_size(64 * PCfg<D, G>::W, 64 * PCfg<D, G>::W))) void attn_prefill_kernel(const PrefParams p) {
     using C = PCfg<D, G>;
     constexpr int W = C::W, ROWS = C::ROWS, BN = C::BN;
@@ -67,55 +65,18 @@ __global__ __attribute__((amdgpu_flat_work_group_size(64 * PCfg<D, G>::W, 64 * P
     constexpr int VS = D + TL_PF_VPAD;   /* V row stride (halves) */
     constexpr float NEG_INF = -__builtin_huge_valf();
 
-    constexpr int K_BYTES = 2 * UNITS * 16, V_BYTES = 2 * BN * VS * 2;
-    __shared__ uint4 s_raw[(K_BYTES + V_BYTES) / 16];
-    uint4 (*const s_k)[UNITS] = (uint4 (*)[UNITS])s_raw;             /* K rows, chunk-swizzled */
-    _Float16 (*const s_v)[BN * VS] =
-        (_Float16 (*)[BN * VS])((unsigned char *)s_raw + K_BYTES);   /* V rows, row-major */
-
-    /* RoPE: (cos, sin) of every pair of a block of rows, built in the tile
-     * memory before the first tile is staged.  A row's table serves all G
-     * heads of the group and both elements of a pair, and powf runs once per
-     * pair and workgroup.  With powf + sincosf per lane and element the
-     * rotation's VALU work bounded every short launch (us per OP_ATTN, before
-     * / after): 333 rows from position 0 at 28/4/128 NEOX 78 / 28.6, 512 rows
-     * at 8/4/256 NEOX and a 1024-key window 131 / 49, 512 rows at 32/8/128
-     * NORM over 32K keys 315 / 290. */
-    constexpr int TS = D / 2 + 2;        /* row stride (pairs): 16 bytes of padding, so the
-                                            16-byte reads of 8 rows cover all banks once */
-    constexpr int TROWS = ROWS * TS * 8 <= K_BYTES + V_BYTES ? ROWS : ROWS / 2;
-    static_assert(TROWS * TS * 8 <= K_BYTES + V_BYTES && TROWS % 32 == 0, "rotation table");
-    static_assert(TL_PF_ROWS * TS * 8 <= K_BYTES + V_BYTES, "rotation table of a unit");
-    float2 *const s_tab = (float2 *)s_raw;
-    __shared__ float s_th[ROPE ? D / 2 : 1];
+    __shared__ uint4 s_k[2][UNITS];                      /* K rows, chunk-swizzled */
+    __shared__ __attribute__((aligned(16))) _Float16 s_v[2][BN * VS];   /* V rows, row-major */
 
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int h = lane >> 5;             /* half-wave */
     const int lr = lane & 31;
 
-    const u32 rpairs = ROPE ? p.rope.rdim >> 1 : 0u;
-    if constexpr (ROPE) {
-        if ((u32)tid < rpairs) s_th[tid] = rope_theta((u32)tid, p.rope.rdim, p.rope.theta);
-    }
-    /* tables of n rows at positions pos0.. (barriers on both sides) */
-    auto rope_tables = [&](u32 pos0, int n) __attribute__((always_inline)) {
-        __syncthreads();   /* the thetas, and the previous table's readers */
-        for (int i = tid; i < n * (D / 2); i += T) {
-            const int row = i / (D / 2), pair = i % (D / 2);
-            if ((u32)pair < rpairs) {
-                float c, s;
-                sincosf((float)(pos0 + (u32)row) * s_th[pair], &s, &c);
-                s_tab[row * TS + pair] = make_float2(c, s);
-            }
-        }
-        __syncthreads();
-    };
-
     /* ---- fused append ----
      * The batch rows go into the cache at the launch's start, before any
      * workgroup reads the cache: workgroup b writes units b, b + grid, ...
-     * (a unit = TL_PF_ROWS rows of one kv-head, the same conversion and
-     * rotation as kv_append_kernel), waits for its stores, and sets the
+     * (a unit = TL_PF_ROWS rows of one kv-head, the same conversion as
+     * kv_append_kernel), waits for its stores, and sets the
      * units' flags to this launch's epoch (below: await_batch).  Stores and
      * flags cross XCDs with the device-coherent policy. */
     const bool fa = !Q8 && p.kin != nullptr;
@@ -126,7 +87,6 @@ __global__ __attribute__((amdgpu_flat_work_group_size(64 * PCfg<D, G>::W, 64 * P
     auto write_unit = [&](u32 kvh_u, u32 r0) __attribute__((always_inline)) {
         const __amdgpu_buffer_rsrc_t rkw = buf_rsrc(p.k), rvw = buf_rsrc(p.v);
         constexpr int IPU = TL_PF_ROWS * CPR;             /* 16-byte items per unit */
-        if constexpr (ROPE) rope_tables(p.pos + r0, TL_PF_ROWS);
         for (int i = tid; i < IPU; i += T) {
             const u32 row = r0 + (u32)(i / CPR), c = (u32)(i % CPR);
             if (row >= p.n) continue;
@@ -135,15 +95,7 @@ __global__ __attribute__((amdgpu_flat_work_group_size(64 * PCfg<D, G>::W, 64 * P
             if (ph >= p.cap) continue;
             const float *kr = p.kin + (u64)row * p.kv_stride + (u64)kvh_u * D;
             const float *vr = p.vin + (u64)row * p.kv_stride + (u64)kvh_u * D;
-            uint4 kk;
-            if constexpr (ROPE) {
-                float t[8];
-                load8_rope_tab(kr, c * 8, p.rope.rdim, p.rope.neox, s_tab + (row - r0) * TS, t);
-                kk = make_uint4(pack_f16x2(t[0], t[1]), pack_f16x2(t[2], t[3]),
-                                pack_f16x2(t[4], t[5]), pack_f16x2(t[6], t[7]));
-            } else {
-                kk = cvt8_f16(kr + c * 8);
-            }
+            const uint4 kk = cvt8_f16(kr + c * 8);
             const uint4 vv = cvt8_f16(vr + c * 8);
             const u32 off = (u32)((((u64)kvh_u * p.cap + ph) * D + c * 8) * 2);
             __builtin_amdgcn_raw_buffer_store_b128(u32x4v_t{kk.x, kk.y, kk.z, kk.w}, rkw, off, 0,
@@ -193,32 +145,34 @@ __global__ __attribute__((amdgpu_flat_work_group_size(64 * PCfg<D, G>::W, 64 * P
     const u32 khi = row_ok ? min(ke, qpos + 1) : 0u;
     const u32 klo = (p.window && qpos + 1 > p.window) ? qpos + 1 - p.window : 0u;
 
-    /* Q operand: lane holds Q[row lr][16s + 8h .. +8] (RoPE'd when p.rope is
-     * set), f16, log2-scaled */
+    /* Q operand: lane holds Q[row lr][16s + 8h .. +8], f16, log2-scaled: from
+     * the f32 rows, or as attn_rope_prep_kernel left it in dst (f16 at the
+     * start of each row's head; this wave alone reads these rows and heads,
+     * before it or the merge writes them) */
     half8_t qop[KS];
-    auto load_q = [&](const float2 *tab) __attribute__((always_inline)) {
+    if (p.q) {
         const float *qrow = p.q + (u64)(row_ok ? my_q : 0) * p.q_stride + (u64)hq * D;
+        const float sc = row_ok ? p.scale_log2 : 0.f;
 #pragma unroll
         for (int s = 0; s < KS; s++) {
-            float t[8];
-            load8_rope_tab(qrow, 16 * s + 8 * h, ROPE ? p.rope.rdim : 0u, p.rope.neox, tab, t);
-            const float sc = row_ok ? p.scale_log2 : 0.f;
-            uint4 u = make_uint4(pack2(t[0] * sc, t[1] * sc), pack2(t[2] * sc, t[3] * sc),
-                                 pack2(t[4] * sc, t[5] * sc), pack2(t[6] * sc, t[7] * sc));
-            qop[s] = h8_from_u4(u);
+            const float4 a = *(const float4 *)(qrow + 16 * s + 8 * h);
+            const float4 b = *(const float4 *)(qrow + 16 * s + 8 * h + 4);
+            qop[s] = h8_from_u4(make_uint4(pack2(a.x * sc, a.y * sc), pack2(a.z * sc, a.w * sc),
+                                           pack2(b.x * sc, b.y * sc), pack2(b.z * sc, b.w * sc)));
         }
-    };
-    if constexpr (ROPE) {
-        /* TROWS rows at a time (all of them but for one head per group) */
-#pragma unroll
-        for (int b = 0; b < ROWS; b += TROWS) {
-            rope_tables(p.pos + qb0 + b, TROWS);
-            if (b <= qsub * 32 && qsub * 32 < b + TROWS) load_q(s_tab + (qsub * 32 - b + lr) * TS);
-        }
-        __syncthreads();   /* the table's readers, before the tiles are staged over it */
     } else {
-        load_q(nullptr);
+        const u16 *qrow = (const u16 *)(p.dst + (u64)(row_ok ? my_q : 0) * p.q_stride + (u64)hq * D);
+#pragma unroll
+        for (int s = 0; s < KS; s++) {
+            const uint4 u = *(const uint4 *)(qrow + 16 * s + 8 * h);
+            qop[s] = row_ok ? h8_from_u4(u) : half8_t{};
+        }
     }
+    /* q is in its registers from here: loads pending at the loop's entry
+     * would make the compiler wait for every load of a tile before its first
+     * MFMA (measured: 322 vs 287 us for 512 rows at 32K keys, 32/8/128) */
+#pragma unroll
+    for (int s = 0; s < KS; s++) __asm__ volatile("" : "+v"(qop[s]));
 
     floatx16_t o[DB];
 #pragma unroll
@@ -529,20 +483,20 @@ __global__ __attribute__((amdgpu_flat_work_group_size(64 * PCfg<D, G>::W, 64 * P
     }
 }
 
-/* One (ROPE, Q8) variant's instances over head_dim {64, 128, 256} x gqa 1..8;
+/* One cache type's instances over head_dim {64, 128, 256} x gqa 1..8;
  * returns the kernel entry point, or NULL for an unsupported shape. */
-#define TL_PREFILL_PICKER(name, ROPE, Q8)                                              \
+#define TL_PREFILL_PICKER(name, Q8)                                                    \
     template <int D>                                                                   \
     static const void *name##_d(int G) {                                               \
         switch (G) {                                                                   \
-        case 1: return (const void *)attn_prefill_kernel<D, 1, ROPE, Q8>;              \
-        case 2: return (const void *)attn_prefill_kernel<D, 2, ROPE, Q8>;              \
-        case 3: return (const void *)attn_prefill_kernel<D, 3, ROPE, Q8>;              \
-        case 4: return (const void *)attn_prefill_kernel<D, 4, ROPE, Q8>;              \
-        case 5: return (const void *)attn_prefill_kernel<D, 5, ROPE, Q8>;              \
-        case 6: return (const void *)attn_prefill_kernel<D, 6, ROPE, Q8>;              \
-        case 7: return (const void *)attn_prefill_kernel<D, 7, ROPE, Q8>;              \
-        case 8: return (const void *)attn_prefill_kernel<D, 8, ROPE, Q8>;              \
+        case 1: return (const void *)attn_prefill_kernel<D, 1, Q8>;                    \
+        case 2: return (const void *)attn_prefill_kernel<D, 2, Q8>;                    \
+        case 3: return (const void *)attn_prefill_kernel<D, 3, Q8>;                    \
+        case 4: return (const void *)attn_prefill_kernel<D, 4, Q8>;                    \
+        case 5: return (const void *)attn_prefill_kernel<D, 5, Q8>;                    \
+        case 6: return (const void *)attn_prefill_kernel<D, 6, Q8>;                    \
+        case 7: return (const void *)attn_prefill_kernel<D, 7, Q8>;                    \
+        case 8: return (const void *)attn_prefill_kernel<D, 8, Q8>;                    \
         default: return nullptr;                                                       \
         }                                                                              \
     }                                                                                  \
@@ -556,6 +510,4 @@ __global__ __attribute__((amdgpu_flat_work_group_size(64 * PCfg<D, G>::W, 64 * P
     }
 
 const void *tl_prefill_fn(int D, int G);            /* tl_prefill.hip */
-const void *tl_prefill_fn_rope(int D, int G);       /* tl_prefill_rope.hip */
 const void *tl_prefill_fn_q8(int D, int G);         /* tl_prefill_q8.hip */
-const void *tl_prefill_fn_q8_rope(int D, int G);    /* tl_prefill_q8_rope.hip */

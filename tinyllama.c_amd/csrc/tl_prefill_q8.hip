@@ -5,4 +5,4 @@
  */
 #include "tl_prefill_kernels.h"
 
-TL_PREFILL_PICKER(tl_prefill_fn_q8, false, true)
+TL_PREFILL_PICKER(tl_prefill_fn_q8, true)

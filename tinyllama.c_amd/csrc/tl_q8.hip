@@ -452,6 +452,12 @@ static int attn_q8(const tl_kv_layer_q8 *L, const tl_attn_args *a, bool append,
      * decode launch quantizes and writes the new rows itself */
     const bool fuse = append && !prefill && a->n <= TL_DEC_MAX_NEW &&
                       (rope.rdim == 0 || a->n <= TL_DEC_Q8_ROPE_NEW);
+    if (prefill && append && rope.rdim) {
+        /* the rotating pre-launch quantizes and writes the new rows */
+        Q8AppendSeg chk;
+        rc = fill_seg_q8(chk, L, a->k, a->v, a->kv_stride, a->slots, a->pos, a->n);
+        return rc ? rc : tl_launch_prefill(lv, a, rope, st, true);
+    }
     if (append && !fuse) {
         rc = append_q8(L, a->k, a->v, a->kv_stride, a->slots, a->pos, a->n, rope, st);
         if (rc) return rc;
