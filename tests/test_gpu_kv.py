@@ -504,6 +504,34 @@ def test_prefill_vs_oracle(T, case, kernel):
     assert e32 < TOL, f"vs f32-cache (reference) oracle {e32}"
 
 
+# (32-row block, q-head) tasks that do not fill the workgroups' waves: one task
+# in the last workgroup, a wave's block before the workgroup's key range ends,
+# a window edge between two blocks, 4 and 8 waves
+PACK_CASES = [
+    # n_head, n_kv, hd, cap, pos, n, window, permuted slots
+    (3, 1, 128, 64, 0, 33, 0, False),
+    (20, 4, 64, 128, 50, 31, 0, True),
+    (14, 2, 128, 256, 130, 65, 70, True),
+    (6, 1, 256, 128, 10, 97, 0, True),
+    (5, 5, 64, 300, 3, 290, 33, False),
+    (64, 64, 64, 600, 0, 520, 0, False),     # 4-wave workgroups exceed the CUs: 8 waves
+    (40, 8, 128, 1100, 600, 460, 200, True),
+]
+
+
+@pytest.mark.parametrize("splits", [0, 1, 2])
+@pytest.mark.parametrize("case", PACK_CASES)
+def test_prefill_task_packing(T, case, splits):
+    import tlkv
+    n_head, n_kv, hd, cap, pos, n, window, perm = case
+    rng = np.random.default_rng(sum(case))
+    slots = (rng.permutation(cap) if perm else np.arange(cap)).astype(np.uint32)
+    with tlkv.tuning(tlkv.TUNE_NO_PREFILL, 2), tlkv.tuning(tlkv.TUNE_PREFILL_SPLITS, splits):
+        out, o16, o32, _, _ = _run_attn(T, n_head, n_kv, hd, cap, pos, n, window, slots, seed=n)
+    assert np.abs(out - o16).max() < TOL
+    assert np.abs(out - o32).max() < TOL
+
+
 def test_prefill_split_invariance(T):
     outs = []
     import tlkv

@@ -100,7 +100,7 @@ struct PrefParams {
     uint32_t cap, ring;
     const float *q;           /* NULL: the rotated f16 q in dst (attn_rope_prep_kernel) */
     float *dst;
-    uint32_t q_stride, pos, n, n_head, n_kv, window;
+    uint32_t q_stride, pos, n, n_head, n_kv, gqa, window;
     float scale_log2;
     uint32_t n_split;
     float *ws_acc;

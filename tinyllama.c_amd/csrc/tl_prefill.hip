@@ -7,9 +7,10 @@
  * the slot table; out = softmax(q.K^T * scale) V.
  *
  * Work decomposition:
- *   A workgroup owns one kv-head, a block of 32*QB query rows and one split
- *   of the key range; its W = G*QB waves each own one q-head of the GQA group
- *   and 32 query rows, so every K/V tile staged in LDS serves G*QB*32 rows.
+ *   A kv-head's work is a list of tasks (32 query rows, one q-head of the GQA
+ *   group); a workgroup owns W consecutive tasks, one per wave, and one split of
+ *   the key range, so every K/V tile staged in LDS serves W*32 query rows and
+ *   every wave has work at any gqa.  W and the split count: plan() below.
  *   Per tile of BN keys (64 at head_dim <= 128, 32 at 256):
  *     S^T[key][row] = K . Q^T      v_mfma_f32_32x32x16_f16 per 32-key block,
  *                                  A = K rows from LDS, B = Q (registers, f16,
@@ -215,10 +216,49 @@ bool tl_use_prefill(const LayerView &L, const tl_attn_args *a) {
     return a->n > TL_DEC_FOLD_MAX_ROWS || (u64)a->n * vis > work;
 }
 
-/* query blocks (one 32-row block per wave and q-head) per workgroup: PCfg::QB */
-static u32 qblocks(u32 D, u32 G) {
-    const u32 wmax = D <= 128 ? 8 : 4;
-    return wmax / G ? wmax / G : 1;
+static u32 task_blocks(u32 n, u32 G, u32 W) { return (G * ((n + 31) / 32) + W - 1) / W; }
+
+/* Waves per workgroup (W) and key splits of a launch, by a cost in us: the
+ * tiles of one workgroup's share of the keys, plus, with splits, the merge
+ * launch and the partials' way through memory (~5 TB/s).  At most one
+ * workgroup per CU counts: a partial second round doubles the time (512 rows
+ * at 28/4/128 over 16K keys: 4 splits 148 us, 5 splits 221).
+ * One tile (64 keys; 32 at head_dim 256) of a workgroup takes 1.70 us with 8
+ * waves and 1.55 with 4 at head_dim 128 (long runs, one workgroup per CU),
+ * 1.18 / 0.94 at 64, 1.75 with 4 at 256, ~2.1 over a Q8_0 cache, where the
+ * dequantization is shared by the workgroup's threads.  So 8 waves read and
+ * stage each key for twice the rows at nearly the same speed and win where
+ * they fill the chip; 4 waves start ~3 us sooner (half the rows to append and
+ * stage) and win below that.  Measured, W = 8 / 4, best split counts (us): 512
+ * rows from position 0 at 32/8/128 27.1 / 23.3, 333 at 28/4/128 23.4 / 18.3,
+ * 512 at 32/8/64 20.5 / 16.0; 333 rows over 1K keys at 32/8/64 21.4 / 19.7;
+ * 100 over 2K 18.7 / 16.6; 512 rows over 4.6K keys at 32/8/128 58.9 / 62.2,
+ * at 32/8/64 39.3 / 40.0; 70 rows over 20K at 28/4/128 52.3 / 53.7. */
+static void plan(const LayerView &L, const tl_attn_args *a, u32 G, u32 cus, u32 &W, u32 &ns) {
+    const u32 D = L.head_dim, bn = D <= 128 ? 64 : 32;
+    const float part_us = (float)a->n * a->n_head * D * 4.f * 2.f / 5e6f;   /* per split */
+    float best = 0.f;
+    W = 0;
+    for (u32 w = D == 256 ? 4 : 8; w >= 4; w -= 4) {
+        const float tile = (L.q8 ? 2.1f : D == 64 ? (w == 8 ? 1.18f : 0.94f)
+                                 : D == 128 ? (w == 8 ? 1.70f : 1.55f) : 1.75f);
+        const u32 base = task_blocks(a->n, G, w) * L.n_kv_head;
+        if (base > cus && W) break;
+        const u32 rows = ((w - 1) / G + 1) * 32;
+        u32 span = a->pos + a->n;              /* most keys any workgroup sees */
+        if (a->window && span > a->window + rows) span = a->window + rows;
+        const u32 most = base < cus ? cus / base : 1u;
+        for (u32 k = 1; k <= most; k++) {
+            const u32 tiles = ((span + k - 1) / k + bn - 1) / bn;
+            const float t = tiles * tile + (w == 8 ? 3.f : 0.f) + (k > 1 ? 5.f + k * part_us : 0.f);
+            if (!W || t < best) {
+                best = t;
+                W = w;
+                ns = k;
+            }
+            if (tiles == 1) break;
+        }
+    }
 }
 
 int tl_launch_prefill(const LayerView &L, const tl_attn_args *a, const RopeCfg &rope,
@@ -252,8 +292,7 @@ int tl_launch_prefill(const LayerView &L, const tl_attn_args *a, const RopeCfg &
         p.q = nullptr;
     }
 
-    const u32 rows = 32 * qblocks(D, G);
-    const u32 nqb = (a->n + rows - 1) / rows;
+    p.gqa = G;
     int cus = 256;
     {
         int dev = 0, n = 0;
@@ -261,12 +300,9 @@ int tl_launch_prefill(const LayerView &L, const tl_attn_args *a, const RopeCfg &
             hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) == hipSuccess && n > 0)
             cus = n;
     }
-    const u32 base = nqb * L.n_kv_head;
-    const u32 span = a->pos + a->n;        /* most keys any workgroup sees */
-    u32 ns = (u32)((cus + base - 1) / base);
-    const u32 max_ns = (span + 511) / 512;  /* keep >= 512 keys per split */
-    if (ns > max_ns) ns = max_ns;
-    if (ns < 1) ns = 1;
+    u32 W, ns;
+    plan(L, a, G, (u32)cus, W, ns);
+    const u32 base = task_blocks(a->n, G, W) * L.n_kv_head;
     if (const u32 t = tl_tune(TL_TUNE_PREFILL_SPLITS)) ns = t;
     if (const size_t fixed = tl_workspace_fixed_acc()) {
         /* no-allocation call: as many key splits as the fixed region holds */
@@ -299,14 +335,14 @@ int tl_launch_prefill(const LayerView &L, const tl_attn_args *a, const RopeCfg &
         }
     }
     const u32 blocks = base * ns;
-    const void *fn = L.q8 ? tl_prefill_fn_q8(D, G) : tl_prefill_fn(D, G);
+    const void *fn = L.q8 ? tl_prefill_fn_q8((int)D, (int)W) : tl_prefill_fn((int)D, (int)W);
     if (!fn) return tl_fail(TL_EINVAL, "prefill: head_dim %u gqa %u", D, G);
     if (rope_on) {
         const int rc = launch_rope_prep(L, a, rope, p.scale_log2, st);
         if (rc) return rc;
     }
     void *args[] = {(void *)&p};
-    HIP_TRY(hipLaunchKernel(fn, dim3(blocks), dim3(64 * G * qblocks(D, G)), args, 0, st));
+    HIP_TRY(hipLaunchKernel(fn, dim3(blocks), dim3(64 * W), args, 0, st));
     if (ns == 1) return TL_OK;
     /* combine the key splits (same partial layout as the decode kernel) */
     DecParams mp;

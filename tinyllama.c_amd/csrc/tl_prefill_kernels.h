@@ -12,15 +12,11 @@
 typedef _Float16 half8_t __attribute__((ext_vector_type(8)));
 typedef float floatx16_t __attribute__((ext_vector_type(16)));
 
-template <int D, int G>
-struct PCfg {
-    static constexpr int WMAX = (D <= 128) ? 8 : 4;
-    static constexpr int QB = (WMAX / G) > 0 ? (WMAX / G) : 1;   /* 32-row query blocks */
-    static constexpr int W = G * QB;                              /* waves */
-    static constexpr int ROWS = 32 * QB;                          /* query rows per WG */
-    static constexpr int BN = (D <= 128) ? 64 : 32;               /* keys per tile */
-};
+/* keys per LDS tile */
+template <int D>
+constexpr int pf_keys() { return D <= 128 ? 64 : 32; }
 
+#define PF_WPE(D) (D == 256 ? 1 : 2)   /* waves per SIMD: 512 or 256 registers */
 #define TL_PF_VPAD 32      /* V row padding in halves: a transpose read's 16-lane
                               group hits 4 rows x 32 B at row steps of 16 (or 48)
                               banks, and the group 32 B to its right fills the
@@ -51,10 +47,9 @@ TL_DEV uint2 ld_tr16(const _Float16 *lds_ptr) {
     return make_uint2(lo, hi);
 }
 
-template <int D, int G, bool Q8>
-__global__ __attribute__((amdgpu_flat_work_group_size(64 * PCfg<D, G>::W, 64 * PCfg<D, G>::W))) void attn_prefill_kernel(const PrefParams p) {
-    using C = PCfg<D, G>;
-    constexpr int W = C::W, ROWS = C::ROWS, BN = C::BN;
+template <int D, int W, bool Q8>
+__global__ __attribute__((amdgpu_flat_work_group_size(64 * W, 64 * W), amdgpu_waves_per_eu(PF_WPE(D)))) void attn_prefill_kernel(const PrefParams p) {
+    constexpr int BN = pf_keys<D>();
     constexpr int T = 64 * W;
     constexpr int CPR = D / 8;           /* 16-byte chunks per row */
     constexpr int KS = D / 16;           /* k-steps of the QK MFMA */
@@ -68,7 +63,8 @@ __global__ __attribute__((amdgpu_flat_work_group_size(64 * PCfg<D, G>::W, 64 * P
     __shared__ uint4 s_k[2][UNITS];                      /* K rows, chunk-swizzled */
     __shared__ __attribute__((aligned(16))) _Float16 s_v[2][BN * VS];   /* V rows, row-major */
 
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int tid = threadIdx.x, lane = tid & 63;
+    const u32 wave = __builtin_amdgcn_readfirstlane((u32)tid >> 6);
     const int h = lane >> 5;             /* half-wave */
     const int lr = lane & 31;
 
@@ -116,25 +112,28 @@ __global__ __attribute__((amdgpu_flat_work_group_size(64 * PCfg<D, G>::W, 64 * P
             __hip_atomic_store(&p.flags[u], epoch, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     }
 
-    /* block -> (K/V range x = kvh * n_split + split, query block); blocks that
-     * read the same K/V range sit on the same XCD (block b runs on XCD b % 8) */
+    /* block -> (K/V range x = kvh * n_split + split, task block); blocks that
+     * read the same K/V range sit on the same XCD (block b runs on XCD b % 8),
+     * the latest rows (the most keys) first */
     const u32 nx = p.n_kv * p.n_split;
-    const u32 x = blockIdx.x % nx, qblk = blockIdx.x / nx;
+    const u32 x = blockIdx.x % nx, tblk = gridDim.x / nx - 1 - blockIdx.x / nx;
     const u32 kvh = x / p.n_split, split = x % p.n_split;
 
-    const int g = wave % G, qsub = wave / G;
-    const u32 hq = kvh * G + g;
-    const u32 qb0 = qblk * ROWS;
-    const u32 my_q = qb0 + qsub * 32 + lr;           /* lane's query row */
+    /* task t of a kv-head = (32-row block t / G, q-head t % G); wave w of the
+     * workgroup has task tblk * W + w, or none past the last */
+    const u32 G = p.gqa, t0 = tblk * W, qb = (t0 + wave) / G;
+    const u32 hq = kvh * G + (t0 + wave) % G;
+    const bool busy = qb * 32 < p.n;
+    const u32 my_q = qb * 32 + lr;                   /* lane's query row */
     const bool row_ok = my_q < p.n;
     const u32 qpos = p.pos + my_q;
     /* the wave's first and last valid query positions */
-    const u32 wq0 = p.pos + qb0 + qsub * 32;
-    const u32 wq1 = p.pos + min(qb0 + qsub * 32 + 31, p.n - 1);
+    const u32 wq0 = p.pos + qb * 32;
+    const u32 wq1 = p.pos + min(qb * 32 + 31, p.n - 1);
 
-    /* key range of the workgroup, then of this split */
-    const u32 wg_last = min(p.pos + qb0 + ROWS, p.pos + p.n);
-    const u32 first_pos = p.pos + qb0;
+    /* key range of the workgroup's rows, then of this split */
+    const u32 wg_last = p.pos + min(((t0 + W - 1) / G + 1) * 32, p.n);
+    const u32 first_pos = p.pos + t0 / G * 32;
     const u32 wg_first = (p.window && first_pos + 1 > p.window) ? first_pos + 1 - p.window : 0;
     const u32 span = wg_last - wg_first;
     u32 chunk = (span + p.n_split - 1) / p.n_split;
@@ -340,6 +339,8 @@ __global__ __attribute__((amdgpu_flat_work_group_size(64 * PCfg<D, G>::W, 64 * P
         }
         const uint4 *sk = s_k[buf];
         const _Float16 *sv_t = s_v[buf];
+        /* tiles past the wave's last row or before its first window: nothing */
+        if (busy && tb <= wq1 && (!p.window || tb + BN + p.window > wq0 + 1)) {
 
         /* S^T - mu = K . Q^T + bias per 32-key block (the accumulators start
          * at -mu, this row's running reference): lane holds keys
@@ -438,6 +439,7 @@ __global__ __attribute__((amdgpu_flat_work_group_size(64 * PCfg<D, G>::W, 64 * P
                 }
             }
         }
+        }
         if (tb + BN < ke) store_tile(buf ^ 1, AHEAD == 2 ? sl ^ 1 : 0);
         __syncthreads();
     };
@@ -483,31 +485,19 @@ __global__ __attribute__((amdgpu_flat_work_group_size(64 * PCfg<D, G>::W, 64 * P
     }
 }
 
-/* One cache type's instances over head_dim {64, 128, 256} x gqa 1..8;
- * returns the kernel entry point, or NULL for an unsupported shape. */
-#define TL_PREFILL_PICKER(name, Q8)                                                    \
-    template <int D>                                                                   \
-    static const void *name##_d(int G) {                                               \
-        switch (G) {                                                                   \
-        case 1: return (const void *)attn_prefill_kernel<D, 1, Q8>;                    \
-        case 2: return (const void *)attn_prefill_kernel<D, 2, Q8>;                    \
-        case 3: return (const void *)attn_prefill_kernel<D, 3, Q8>;                    \
-        case 4: return (const void *)attn_prefill_kernel<D, 4, Q8>;                    \
-        case 5: return (const void *)attn_prefill_kernel<D, 5, Q8>;                    \
-        case 6: return (const void *)attn_prefill_kernel<D, 6, Q8>;                    \
-        case 7: return (const void *)attn_prefill_kernel<D, 7, Q8>;                    \
-        case 8: return (const void *)attn_prefill_kernel<D, 8, Q8>;                    \
-        default: return nullptr;                                                       \
-        }                                                                              \
-    }                                                                                  \
-    const void *name(int D, int G) {                                                   \
-        switch (D) {                                                                   \
-        case 64: return name##_d<64>(G);                                               \
-        case 128: return name##_d<128>(G);                                             \
-        case 256: return name##_d<256>(G);                                             \
-        default: return nullptr;                                                       \
-        }                                                                              \
+/* One cache type's instances: head_dim {64, 128, 256} x waves per workgroup
+ * (tl_prefill.hip); NULL for a shape without one. */
+#define TL_PREFILL_PICKER(name, Q8)                                                          \
+    const void *name(int D, int W) {                                                         \
+        switch (D) {                                                                         \
+        case 64: return W == 8 ? (const void *)attn_prefill_kernel<64, 8, Q8>                \
+                      : W == 4 ? (const void *)attn_prefill_kernel<64, 4, Q8> : nullptr;     \
+        case 128: return W == 8 ? (const void *)attn_prefill_kernel<128, 8, Q8>              \
+                       : W == 4 ? (const void *)attn_prefill_kernel<128, 4, Q8> : nullptr;   \
+        case 256: return W == 4 ? (const void *)attn_prefill_kernel<256, 4, Q8> : nullptr;   \
+        default: return nullptr;                                                             \
+        }                                                                                    \
     }
 
-const void *tl_prefill_fn(int D, int G);            /* tl_prefill.hip */
-const void *tl_prefill_fn_q8(int D, int G);         /* tl_prefill_q8.hip */
+const void *tl_prefill_fn(int D, int W);            /* tl_prefill.hip */
+const void *tl_prefill_fn_q8(int D, int W);         /* tl_prefill_q8.hip */
