@@ -70,6 +70,8 @@ static u32 tuned(int key, u32 dflt) {
     return v ? v : dflt;
 }
 
+static u32 umax(u32 a, u32 b) { return a > b ? a : b; }
+
 /* CUs of the current device (cached per device; launches from several host
  * threads may fill the cache at once and store the same value) */
 static int cu_count() {
@@ -90,8 +92,8 @@ static int cu_count() {
  * lock: several host threads may launch at once) */
 static int resident_per_cu(const void *fn, int threads) {
     static std::mutex mu;
-    static const void *keys[64];
-    static int vals[64];
+    static const void *keys[512];
+    static int vals[512];
     static int n = 0;
     {
         std::lock_guard<std::mutex> lk(mu);
@@ -101,7 +103,7 @@ static int resident_per_cu(const void *fn, int threads) {
     int b = 0;
     if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&b, fn, threads, 0) != hipSuccess || b < 1) b = 1;
     std::lock_guard<std::mutex> lk(mu);
-    if (n < 64) {
+    if (n < 512) {
         keys[n] = fn;
         vals[n++] = b;
     }
@@ -122,15 +124,6 @@ static int launch_decode(DecParams &p, u32 n_rows_total, u32 head_dim, u32 G, u3
                                           "at most %d rows", TL_DEC_Q8_ROPE_NEW);
     }
     DecKernel K;
-    /* tiles on the matrix cores where measured faster (8 kv-heads, 1K and
-     * 32K keys, gqa 1-8): the f16 cache at head_dim 64 and 128 from gqa 2
-     * (gqa 8: 16.3 vs 38.3 us at 32K keys; gqa 1 even); the Q8_0 cache at
-     * head_dim 64 from gqa 2 and at 128 from gqa 4 (gqa 8: 26.9 vs 57.9 us;
-     * with two ring tiles per softmax chain the matrix tile takes 24.3 vs
-     * 24.65 us at gqa 4 and 8 kv-heads, 16.4 vs 17.9 at 4 kv-heads; gqa 1
-     * stays on the vector tile: 17.7 vs 25.9 us).  At head_dim 256 (8-key
-     * tiles, half of each 16-key block padding) the vector tile is faster
-     * (config 5, gqa 2: 13.1 vs 13.4 us per launch). */
     const u32 tile_sel = tl_tune(TL_TUNE_DECODE_MFMA);
     /* with several batch rows the matrix tile folds up to 16 / gqa of them
      * (8 / gqa at head_dim 256) into its columns and reads K/V once for all,
@@ -143,8 +136,7 @@ static int launch_decode(DecParams &p, u32 n_rows_total, u32 head_dim, u32 G, u3
     const u32 rmax = (head_dim == 256 ? 8u : 16u) / G;
     const bool can_fold = fold_rows && rows_in > 1 && rmax > 1 &&
                           !tl_tune(TL_TUNE_DECODE_MERGE_KERNEL) && tl_tune(TL_TUNE_DECODE_ROWS) != 1;
-    const bool mf_auto = can_fold ||
-                         (head_dim == 64 ? G >= 2 : head_dim == 128 ? G >= (q8 ? 4u : 2u) : false);
+    const bool mf_auto = can_fold || tl_decode_matrix_tile((int)head_dim, (int)G, q8);
     const bool mf = tile_sel == 2 || (tile_sel != 1 && mf_auto);
     switch (head_dim) {
     case 64: K = pick_kernel<64>((int)G, p.rope.rdim != 0, q8, mf); break;
@@ -179,14 +171,20 @@ static int launch_decode(DecParams &p, u32 n_rows_total, u32 head_dim, u32 G, u3
      * for them) */
     u32 n_split = n_groups < target ? (u32)(target / n_groups) : 1u;
     const u32 waves = (u32)K.threads / 64;
-    /* fewest keys per split: a tile for every wave at head_dim 128, for half
-     * of them at 64 and 256, at most 128 keys (measured: head_dim 64, P =
-     * 700: 128 keys per split 8.8 us vs 9.5 us at 256, and fewer make the
-     * merge dearer than the shorter chunks save; head_dim 256, the 1024-key
-     * window of config 5's local layers: 32 keys 12.1 us per launch on
-     * average vs 12.55 at 64) */
-    const u32 min_tiles = head_dim == 128 ? waves : waves / 2;
-    const u32 min_keys = tuned(TL_TUNE_DECODE_MIN_KEYS, min_tiles * tk < 128 ? min_tiles * tk : 128);
+    /* fewest keys per split: a tile for half of the waves, at most 128 keys; at
+     * head_dim 128 only up to as many splits as one trip of the merge folds
+     * (8), then 128.  Measured, us per launch: head_dim 64, 700 keys: 128 keys
+     * per split 8.2, 64 9.0, 256 8.9; 128, 700 keys of 8 kv-heads: 64 keys 8.8,
+     * 128 9.2; of 4 kv-heads over 500 keys 8.6 / 9.5 (Q8_0 9.5 / 10.6), over
+     * 1100 10.7 / 10.1, 94 keys 8.4 / 6.9; 256, a 1024-key window: 32 keys 9.4,
+     * 128 10.4 */
+    const u32 one_trip = 8;
+    const u32 half_waves = waves / 2 * tk;
+    u32 min_keys = tuned(TL_TUNE_DECODE_MIN_KEYS, half_waves);
+    if (head_dim == 128 && !tl_tune(TL_TUNE_DECODE_MIN_KEYS)) {
+        const u32 c = (max_vis + one_trip - 1) / one_trip;
+        min_keys = max_vis <= 128 || c > 128 ? 128 : umax(c, half_waves);
+    }
     const u32 max_split = (max_vis + min_keys - 1) / min_keys;
     /* keys per workgroup: limited by the slot-table staging only (u32
      * indices, or u16 ones in the matrix-core f16 instances when every
@@ -214,8 +212,52 @@ static int launch_decode(DecParams &p, u32 n_rows_total, u32 head_dim, u32 G, u3
         }
     }
     if (n_split < 1) n_split = 1;
-    const u32 chunk = (max_vis + n_split - 1) / n_split;
+    u32 chunk = (max_vis + n_split - 1) / n_split;
     n_split = (max_vis + chunk - 1) / chunk;
+    /* sessions of unequal lengths: split counts by length, from the smallest
+     * chunk whose workgroups still fit the rounds that the equal split takes
+     * (its workgroups of the short sessions would have no keys, while the long
+     * sessions' had max_vis / n_split).  8 sessions of 512 to 8192 keys at
+     * 28/4/128: 21.4 us per launch with equal counts, 17.7 by length. */
+    p.ragged = 0;
+    u64 grid = (u64)n_split * n_groups;
+    if (rows == 1 && n_rows_total > 1 && n_split > 1 &&
+        mf == tl_decode_matrix_tile((int)head_dim, (int)G, q8)) {
+        const u32 n_seq = n_rows_total;
+        u32 vis[TL_MAX_BATCH_SEQ];
+        for (u32 i = 0; i < n_seq; i++) {
+            const u32 nk = p.seq[i].pos + 1;
+            vis[i] = (p.window && nk > p.window) ? p.window : nk;
+        }
+        auto wgs = [&](u32 c) {
+            u64 t = 0;
+            for (u32 i = 0; i < n_seq; i++) t += (vis[i] + c - 1) / c;
+            return t * p.n_kv;
+        };
+        const u64 room = grid > target ? (grid + target - 1) / target * target : target;
+        u32 lo = min_keys < chunk ? min_keys : chunk, hi = chunk;
+        while (lo < hi) {
+            const u32 mid = (lo + hi) / 2;
+            if (wgs(mid) <= room) hi = mid;
+            else lo = mid + 1;
+        }
+        const u32 most = (max_vis + hi - 1) / hi;
+        /* worth it from a sixth fewer keys on */
+        if (hi <= chunk - chunk / 6 && (!any_staged || hi <= TL_DEC_MAX_CHUNK) && most <= TL_MERGE_MAX_SPLIT_DIST && G * most <= 2048 &&
+            n_groups <= TL_MERGE_MAX_GROUPS && !tl_tune(TL_TUNE_DECODE_MERGE_KERNEL)) {
+            p.ragged = 1;
+            chunk = hi;
+            n_split = most;
+            u32 w = 0;
+            for (u32 i = 0; i <= TL_MAX_BATCH_SEQ; i++) {
+                p.wg0[i] = i <= n_seq ? w : 0xffffffffu;
+                if (i < n_seq) w += (vis[i] + chunk - 1) / chunk * p.n_kv;
+            }
+            grid = w;
+            K = q8 ? tl_pick_decode_rag_q8((int)head_dim, (int)G, p.rope.rdim != 0)
+                   : tl_pick_decode_rag((int)head_dim, (int)G, p.rope.rdim != 0);
+        }
+    }
     if (n_split > TL_MERGE_MAX_SPLIT)
         return tl_fail(TL_EINVAL, "decode: %u keys need %u splits", max_vis, n_split);
     p.chunk = chunk;
@@ -238,15 +280,24 @@ static int launch_decode(DecParams &p, u32 n_rows_total, u32 head_dim, u32 G, u3
     }
     p.rows_per_wg = R;
     if (n_split > 1) {
-        /* every split merges a slice of the output (dist) when there are
-         * enough splits to share the merge (measured: with 8 or fewer the
-         * last split alone is faster) and all of the grid is resident at
+        /* slices (dist): tl_internal.h; only with all of the grid resident at
          * once (a split waits, bounded, for the rest of its group) */
         const u64 resident = (u64)resident_per_cu(K.fn, K.threads) * cu_count();
-        p.dist = in_kernel_merge && n_split >= 12 && n_split <= TL_MERGE_MAX_SPLIT_DIST &&
-                 (u64)n_split * n_groups <= resident && !tl_tune(TL_TUNE_DECODE_SINGLE_MERGE);
+        const u32 cols4 = R * G * head_dim / 4;      /* output float4s of a group */
+        u32 dist_min = TL_MERGE_MIN_SPLIT_DIST;
+        dist_min = umax(dist_min, (TL_MERGE_MIN_BYTES_DIST + cols4 * 16 - 1) / (cols4 * 16));
+        dist_min = umax(dist_min, (cols4 + TL_MERGE_SLICE_MAX - 1) / TL_MERGE_SLICE_MAX);
+        p.dist = in_kernel_merge && n_split >= dist_min && n_split <= TL_MERGE_MAX_SPLIT_DIST &&
+                         grid <= resident && !tl_tune(TL_TUNE_DECODE_SINGLE_MERGE)
+                     ? dist_min : 0u;
+        p.dist_groups = (u32)n_groups;
+        if (p.ragged) {
+            p.dist_groups = 0;
+            for (u32 i = 0; i < n_rows_total; i++)
+                if (p.wg0[i + 1] - p.wg0[i] >= dist_min * p.n_kv) p.dist_groups += p.n_kv;
+        }
         TlWorkspace *w;
-        size_t parts = (size_t)n_groups * R * G * n_split;
+        size_t parts = (size_t)grid * R * G;
         /* dist: one (m, l, epoch, ~epoch) record of 16 bytes per partial */
         int rc = tl_workspace_get(st, parts * head_dim, p.dist ? 2 * parts : parts,
                                   in_kernel_merge ? TL_MERGE_CNT_WORDS : 0, &w);
@@ -260,7 +311,7 @@ static int launch_decode(DecParams &p, u32 n_rows_total, u32 head_dim, u32 G, u3
         }
     }
     void *args[] = {(void *)&p};
-    HIP_TRY(hipLaunchKernel(K.fn, dim3(n_split * (u32)n_groups), dim3(K.threads), args, 0, st));
+    HIP_TRY(hipLaunchKernel(K.fn, dim3((u32)grid), dim3(K.threads), args, 0, st));
     if (n_split == 1 || in_kernel_merge) return TL_OK;
     return tl_launch_merge(p, n_rows_total, head_dim, st);
 }

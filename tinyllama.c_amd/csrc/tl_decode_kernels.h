@@ -668,91 +668,137 @@ TL_DEV void mfma_tile_q8(uint4 *stage, const u16 *scl, const dh8_t (&qb)[D / 32]
 
 constexpr int pow2_floor(int x) { return x >= 16 ? 16 : x >= 8 ? 8 : x >= 4 ? 4 : x >= 2 ? 2 : 1; }
 
-/* Merge of a group's n_split partials by its last workgroup, in registers:
- * TPC threads per output float4 (h, d..d+3) each fold their share of the
- * splits with an online max, then combine across the TPC lanes with DPP:
- * out = sum_s exp2(m_s - M) acc_s / sum_s exp2(m_s - M) l_s.  The first
- * batch of partial rows and every (m, l) pair are requested together
- * (device-coherent loads); the pairs go through LDS (s_ml: G*n_split). */
-template <int D, int G, int NT>
-TL_DEV void split_merge_regs(const DecParams &p, u32 pb, u32 kvh, u32 r, u32 gh, u32 ncol,
-                             const DecSeq &sq, float2 *s_ml) {
+/* Merge of a group's ns partials by its last workgroup:
+ * out = sum_s exp2(m_s - M) acc_s / sum_s exp2(m_s - M) l_s per output float4
+ * (head h, dims d..d+3; ncol heads, ncol * D/4 <= NT float4s).  Bound by the
+ * round trips of its device-coherent loads.  Few float4s and many splits: the
+ * threads cover the float4s P times over (P shares of the splits, consecutive
+ * lanes on consecutive 16 bytes of one split's row), so all rows are requested
+ * in one trip, one wave per head turns the (m, l) pairs into weights meanwhile,
+ * and the shares add through LDS.  Otherwise each thread folds all splits with
+ * an online max, K rows per trip.  us per launch, shares / fold: 32 splits of
+ * 4 heads at head_dim 128 over 32K keys 28.1 / 28.5, over 4K 10.2 / 10.6; of 2
+ * heads at 256 9.4 / 9.6; but 32 splits of 7 heads at 128 (P = 2) 10.6 / 10.1,
+ * and 16 splits of 4 heads at 64 9.2 / 8.7 (two trips fold them).
+ * s_buf: ncol * ns <= 2048 pairs, then the shares. */
+template <int D, int NT>
+TL_DEV void split_merge_regs(const DecParams &p, u32 pb, const float2 *ml_g, u32 ns, u32 kvh,
+                             u32 r, u32 gh, u32 ncol, const DecSeq &sq, float2 *s_buf) {
     constexpr float NEG_INF = -__builtin_huge_valf();
-    constexpr int COLS_MAX = G * D / 4;
-    const int COLS = (int)ncol * (D / 4);
-    constexpr int TPC = pow2_floor(NT / COLS_MAX > 16 ? 16 : (NT / COLS_MAX < 1 ? 1 : NT / COLS_MAX));
-    constexpr int K = 8;                       /* splits per load batch */
-    const int tid = threadIdx.x;
-    const u32 ns = p.n_split;
-    const __amdgpu_buffer_rsrc_t rml = buf_rsrc(p.ws_ml + pb);
+    constexpr u32 K = 8;                       /* splits per load batch */
+    const u32 tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const u32 COLS = ncol * (D / 4);
+    const u32 P = ns > 2 * K && COLS <= NT / 4 ? (u32)NT / COLS : 1u;
+    const u32 part = (tid / (D / 4)) / ncol, h = (tid / (D / 4)) % ncol, d = (tid % (D / 4)) * 4;
+    const __amdgpu_buffer_rsrc_t rml = buf_rsrc(ml_g);
     const __amdgpu_buffer_rsrc_t racc = buf_rsrc(p.ws_acc + (u64)pb * D);
-    const int part = tid % TPC;
-    const int col0 = tid / TPC;
+    float *const s_inv = (float *)(s_buf + 2048);
+    float4 *const s_o = (float4 *)(s_inv + 64);
     u32x4v_t a[K];
-    auto load_batch = [&](int col, u32 s0) {
-        const int h = col / (D / 4), d = (col % (D / 4)) * 4;
+    auto load_batch = [&](u32 s0) __attribute__((always_inline)) {
 #pragma unroll
-        for (int k = 0; k < K; k++) {
-            const u32 s = min(s0 + k * TPC, ns - 1);
-            const u32 off = (((u32)h * ns + s) * D + d) * 4;
-            a[k] = __builtin_amdgcn_raw_buffer_load_b128(racc, off, 0, TL_SC1);
+        for (u32 k = 0; k < K; k++) {
+            const u32 s = min(s0 + k * P, ns - 1);
+            a[k] = __builtin_amdgcn_raw_buffer_load_b128(racc, ((h * ns + s) * D + d) * 4, 0, TL_SC1);
         }
     };
-    if (col0 < COLS) load_batch(col0, (u32)part);
-    for (u32 i = tid; i < ncol * ns; i += NT) {
-        const u32x2v_t ml = __builtin_amdgcn_raw_buffer_load_b64(rml, i * 8, 0, TL_SC1);
-        s_ml[i] = make_float2(__uint_as_float(ml[0]), __uint_as_float(ml[1]));
-    }
-    __asm__ volatile("s_waitcnt vmcnt(0)" ::: "memory");
-    __syncthreads();
-    for (int col = col0; col < COLS; col += NT / TPC) {
-        const int h = col / (D / 4), d = (col % (D / 4)) * 4;
-        const float2 *mlh = s_ml + (u32)h * ns;
-        float M = NEG_INF, L = 0.f;
-        float4 O = make_float4(0.f, 0.f, 0.f, 0.f);
-        for (u32 s0 = part; s0 < ns; s0 += K * TPC) {
-            if (col != col0 || s0 != (u32)part) load_batch(col, s0);
-            float2 ml[K];
-            float bm = NEG_INF;
-#pragma unroll
-            for (int k = 0; k < K; k++) {
-                const u32 s = s0 + k * TPC;
-                ml[k] = mlh[min(s, ns - 1)];
-                if (s >= ns) ml[k] = make_float2(NEG_INF, 0.f);   /* past the last split */
-                bm = fmaxf(bm, ml[k].x);
+    float4 O = make_float4(0.f, 0.f, 0.f, 0.f);
+    float inv = 0.f;
+    if (P > 1) {
+        auto pair = [&](u32 hh, u32 s) {
+            const u32x2v_t v = __builtin_amdgcn_raw_buffer_load_b64(rml, (hh * ns + min(s, ns - 1)) * 8, 0, TL_SC1);
+            return make_float2(s < ns ? __uint_as_float(v[0]) : NEG_INF, __uint_as_float(v[1]));
+        };
+        float2 ml0 = make_float2(NEG_INF, 0.f);
+        if (wave < ncol) ml0 = pair(wave, lane);
+        if (part < P) load_batch(part);
+        float *const s_w = (float *)s_buf;
+        for (u32 hh = wave; hh < ncol; hh += NT / 64) {
+            float2 ml = hh == wave ? ml0 : pair(hh, lane);
+            float M = ml.x;
+            for (u32 s = lane + 64; s < ns; s += 64) M = fmaxf(M, pair(hh, s).x);
+            M = group_max<64>(M);
+            const float mu = (M == NEG_INF) ? 0.f : M;
+            float L = 0.f;
+            for (u32 s = lane; s < ns; s += 64) {
+                if (s != lane) ml = pair(hh, s);
+                const float w = fast_exp2(ml.x - mu);
+                s_w[hh * ns + s] = w;
+                L = fmaf(w, ml.y, L);
             }
-            const float nm = fmaxf(M, bm);
-            const float mu = (nm == NEG_INF) ? 0.f : nm;
-            const float sc = fast_exp2(M - mu);
-            L *= sc;
-            O.x *= sc; O.y *= sc; O.z *= sc; O.w *= sc;
-            M = nm;
+            L = group_sum<64>(L);
+            if (lane == 0) s_inv[hh] = 1.0f / L;
+        }
+        __syncthreads();
+        if (part < P) {
+            for (u32 s0 = part; s0 < ns; s0 += K * P) {
+                if (s0 != part) load_batch(s0);
 #pragma unroll
-            for (int k = 0; k < K; k++) {
-                const float w = fast_exp2(ml[k].x - mu);
-                L = fmaf(w, ml[k].y, L);
-                O.x = fmaf(w, __uint_as_float(a[k][0]), O.x);
-                O.y = fmaf(w, __uint_as_float(a[k][1]), O.y);
-                O.z = fmaf(w, __uint_as_float(a[k][2]), O.z);
-                O.w = fmaf(w, __uint_as_float(a[k][3]), O.w);
+                for (u32 k = 0; k < K; k++) {
+                    const u32 s = s0 + k * P;
+                    if (s < ns) {
+                        const float w = s_w[h * ns + s];
+                        O.x = fmaf(w, __uint_as_float(a[k][0]), O.x);
+                        O.y = fmaf(w, __uint_as_float(a[k][1]), O.y);
+                        O.z = fmaf(w, __uint_as_float(a[k][2]), O.z);
+                        O.w = fmaf(w, __uint_as_float(a[k][3]), O.w);
+                    }
+                }
             }
+            if (part) s_o[tid] = O;
         }
-        if constexpr (TPC > 1) {
-            const float Mg = group_max<TPC>(M);
-            const float mu = (Mg == NEG_INF) ? 0.f : Mg;
-            const float e = fast_exp2(M - mu);
-            L = group_sum<TPC>(L * e);
-            O.x = group_sum<TPC>(O.x * e);
-            O.y = group_sum<TPC>(O.y * e);
-            O.z = group_sum<TPC>(O.z * e);
-            O.w = group_sum<TPC>(O.w * e);
-        }
+        __syncthreads();
         if (part == 0) {
-            const float inv = 1.0f / L;
-            *(float4 *)&sq.dst[(u64)(r + h / gh) * p.q_stride + (u64)(kvh * gh + h % gh) * D + d] =
-                make_float4(O.x * inv, O.y * inv, O.z * inv, O.w * inv);
+            for (u32 q = 1; q < P; q++) {
+                const float4 t = s_o[tid + q * COLS];
+                O.x += t.x; O.y += t.y; O.z += t.z; O.w += t.w;
+            }
+            inv = s_inv[h];
+        }
+    } else {
+        if (part == 0) load_batch(0);
+        for (u32 i = tid; i < ncol * ns; i += NT) {
+            const u32x2v_t ml = __builtin_amdgcn_raw_buffer_load_b64(rml, i * 8, 0, TL_SC1);
+            s_buf[i] = make_float2(__uint_as_float(ml[0]), __uint_as_float(ml[1]));
+        }
+        __asm__ volatile("s_waitcnt vmcnt(0)" ::: "memory");
+        __syncthreads();
+        if (part == 0) {
+            float M = NEG_INF, L = 0.f;
+            const float2 *mlh = s_buf + h * ns;
+            for (u32 s0 = 0; s0 < ns; s0 += K) {
+                if (s0) load_batch(s0);
+                float2 ml[K];
+                float bm = NEG_INF;
+#pragma unroll
+                for (u32 k = 0; k < K; k++) {
+                    const u32 s = s0 + k;
+                    ml[k] = mlh[min(s, ns - 1)];
+                    if (s >= ns) ml[k] = make_float2(NEG_INF, 0.f);   /* past the last split */
+                    bm = fmaxf(bm, ml[k].x);
+                }
+                const float nm = fmaxf(M, bm);
+                const float mu = (nm == NEG_INF) ? 0.f : nm;
+                const float sc = fast_exp2(M - mu);
+                L *= sc;
+                O.x *= sc; O.y *= sc; O.z *= sc; O.w *= sc;
+                M = nm;
+#pragma unroll
+                for (u32 k = 0; k < K; k++) {
+                    const float w = fast_exp2(ml[k].x - mu);
+                    L = fmaf(w, ml[k].y, L);
+                    O.x = fmaf(w, __uint_as_float(a[k][0]), O.x);
+                    O.y = fmaf(w, __uint_as_float(a[k][1]), O.y);
+                    O.z = fmaf(w, __uint_as_float(a[k][2]), O.z);
+                    O.w = fmaf(w, __uint_as_float(a[k][3]), O.w);
+                }
+            }
+            inv = 1.0f / L;
         }
     }
+    if (part == 0)
+        *(float4 *)&sq.dst[(u64)(r + h / gh) * p.q_stride + (u64)(kvh * gh + h % gh) * D + d] =
+            make_float4(O.x * inv, O.y * inv, O.z * inv, O.w * inv);
 }
 
 /* Bounded waits of the in-launch split merge (polls of device-coherent
@@ -767,11 +813,10 @@ TL_DEV void split_merge_regs(const DecParams &p, u32 pb, u32 kvh, u32 r, u32 gh,
  * w_s = exp2(m_s - max m).  Partial rows and their (m, l, epoch) records
  * (float4 per partial) are read with device-coherent loads. */
 template <int D, int W>
-TL_DEV void merge_slice(const DecParams &p, u32 pb, u32 r, u32 kvh, u32 gh, u32 ncol,
+TL_DEV void merge_slice(const DecParams &p, u32 pb, u32 ns, u32 r, u32 kvh, u32 gh, u32 ncol,
                         const DecSeq &sq, u32 slice, u32 cps) {
     constexpr float NEG_INF = -__builtin_huge_valf();
     const u32 COLS = ncol * (D / 4);
-    const u32 ns = p.n_split;
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const u32 c0 = slice * cps, c1 = min(c0 + cps, COLS);
     const __amdgpu_buffer_rsrc_t rrec = buf_rsrc((const float4 *)p.ws_ml + pb);
@@ -816,7 +861,7 @@ TL_DEV void merge_slice(const DecParams &p, u32 pb, u32 r, u32 kvh, u32 gh, u32 
  * the rows staged from the f32 input. */
 #define TL_RING_WAVES 8
 #define TL_RING_STAGES 2
-template <int D, int G, bool ROPE, bool Q8, bool MF, bool S16>
+template <int D, int G, bool ROPE, bool Q8, bool MF, bool S16, bool RAGGED>
 __device__ __attribute__((always_inline)) inline void decode_ring_body(const DecParams &p) {
     using C = RCfg<D>;
     constexpr int LPK = C::LPK, CPR = C::CPR, TK = C::TK, UNITS = C::UNITS, LD = C::LD;
@@ -861,18 +906,31 @@ __device__ __attribute__((always_inline)) inline void decode_ring_body(const Dec
         buf_rsrc(p.dist ? p.counters + TL_MERGE_LAUNCHES : nullptr), p.dist ? 0u : 0xfffffff0u, 0,
         TL_SC1);                                   /* without dist: out of range, reads 0 */
 
-    const u32 n_split = p.n_split;
-    const u32 n_groups = gridDim.x / n_split;
+    u32 n_split = p.n_split;
     const u32 bid = blockIdx.x;
-    u32 grp, split;
-    if ((n_groups & 7) == 0) {
-        const u32 xcd = bid & 7, local = bid >> 3;
-        grp = xcd + 8 * (local / n_split);
+    u32 grp, split, wg_grp;   /* group, split, the group's first workgroup (partials) */
+    if constexpr (RAGGED) {
+        u32 s = 0;
+#pragma unroll
+        for (u32 i = 1; i < TL_MAX_BATCH_SEQ; i++) s += bid >= p.wg0[i] ? 1u : 0u;
+        const u32 w0 = p.wg0[s], local = bid - w0;
+        n_split = (p.wg0[s + 1] - w0) / p.n_kv;
         split = local % n_split;
+        grp = s * p.n_kv + local / n_split;
+        wg_grp = bid - split;
     } else {
-        grp = bid / n_split;
-        split = bid % n_split;
+        const u32 n_groups = gridDim.x / n_split;
+        if ((n_groups & 7) == 0) {
+            const u32 xcd = bid & 7, local = bid >> 3;
+            grp = xcd + 8 * (local / n_split);
+            split = local % n_split;
+        } else {
+            grp = bid / n_split;
+            split = bid % n_split;
+        }
+        wg_grp = grp * n_split;
     }
+    const bool dist = p.dist && (!RAGGED || n_split >= p.dist);
     /* group = (session, block of R batch rows, kv-head); R > 1 only with the
      * matrix-core tile.  The group's keys run from its first row's window
      * start to its last row's last key; each column masks its own row's. */
@@ -1373,7 +1431,9 @@ __device__ __attribute__((always_inline)) inline void decode_ring_body(const Dec
     const bool last_merges = p.counters != nullptr;
     /* the group's partials: [column][split][D] from pb (R = 1: the layout
      * attn_merge_kernel reads, [row][head][split][D]) */
-    const u32 pb = grp * (R * G) * n_split;
+    const u32 pb = wg_grp * (R * G);
+    /* its (max, sum) pairs; a launch with dist keeps 16 bytes per partial */
+    float2 *const ml_g = p.ws_ml + (p.dist ? 2 : 1) * (u64)pb;
     __shared__ float2 s_rec[CGT];
     /* output float4 (column h = batch row of the group x G + head, dims
      * d..d+3) of the workgroup's state: the result itself (one split) or
@@ -1393,12 +1453,12 @@ __device__ __attribute__((always_inline)) inline void decode_ring_body(const Dec
                          __float_as_uint(O.w)},
                 buf_rsrc(p.ws_acc + (u64)pb * D), (pi * D + d) * 4, 0, TL_SC1);
             if (d == 0) {
-                if (p.dist)
+                if (dist)
                     s_rec[h] = make_float2(mm, L);   /* record written below */
                 else
                     __builtin_amdgcn_raw_buffer_store_b64(
                         u32x2v_t{__float_as_uint(mm), __float_as_uint(L)},
-                        buf_rsrc(p.ws_ml + pb), pi * 8, 0, TL_SC1);
+                        buf_rsrc(ml_g), pi * 8, 0, TL_SC1);
             }
         } else {
             const u64 pi = ((u64)gblk * p.n_head + hq) * n_split + split;
@@ -1584,7 +1644,7 @@ __device__ __attribute__((always_inline)) inline void decode_ring_body(const Dec
     __asm__ volatile("s_waitcnt vmcnt(0)" ::: "memory");
     __syncthreads();
     u32 *arrive = p.counters + grp * TL_MERGE_PAD;
-    if (p.dist) {
+    if (dist) {
         __shared__ u32 s_epoch;
         if (tid == 0) s_epoch = launches + 1u;
         __syncthreads();
@@ -1592,7 +1652,7 @@ __device__ __attribute__((always_inline)) inline void decode_ring_body(const Dec
         const u32 COLS = cg * (D / 4);
         const u32 cps = (COLS + n_split - 1) / n_split;   /* columns per slice */
         const u32 c0 = split * cps, c1 = min(c0 + cps, COLS);
-        const __amdgpu_buffer_rsrc_t rrec = buf_rsrc((const float4 *)p.ws_ml + pb);
+        const __amdgpu_buffer_rsrc_t rrec = buf_rsrc(ml_g);
         if ((u32)tid < cg) {
             const u32 pi = (u32)tid * n_split + split;
             __builtin_amdgcn_raw_buffer_store_b128(
@@ -1631,7 +1691,7 @@ __device__ __attribute__((always_inline)) inline void decode_ring_body(const Dec
             if (tid == 0)
                 __hip_atomic_store(&tags[split], epoch, __ATOMIC_RELAXED,
                                    __HIP_MEMORY_SCOPE_AGENT);
-            merge_slice<D, W>(p, pb, r, kvh, G, cg, sq, split, cps);
+            merge_slice<D, W>(p, pb, n_split, r, kvh, G, cg, sq, split, cps);
             return;
         }
         if (tid == 0) {
@@ -1643,14 +1703,14 @@ __device__ __attribute__((always_inline)) inline void decode_ring_body(const Dec
              * otherwise see the next one and make its peers' polls time out) */
             const u32 closed = __hip_atomic_fetch_add(p.counters + TL_MERGE_CLOSED, 1u,
                                                       __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-            if (closed == n_groups - 1) {
+            if (closed == p.dist_groups - 1) {
                 __hip_atomic_store(p.counters + TL_MERGE_CLOSED, 0u, __ATOMIC_RELAXED,
                                    __HIP_MEMORY_SCOPE_AGENT);
                 __hip_atomic_fetch_add(p.counters + TL_MERGE_LAUNCHES, 1u, __ATOMIC_RELAXED,
                                        __HIP_MEMORY_SCOPE_AGENT);
             }
         }
-        merge_slice<D, W>(p, pb, r, kvh, G, cg, sq, split, cps);
+        merge_slice<D, W>(p, pb, n_split, r, kvh, G, cg, sq, split, cps);
         /* slices whose owner has not claimed them (yet) */
         if (wave == 0) {
             u64 todo = 0;
@@ -1668,7 +1728,7 @@ __device__ __attribute__((always_inline)) inline void decode_ring_body(const Dec
         }
         __syncthreads();
         for (u64 todo = s_todo; todo; todo &= todo - 1)
-            merge_slice<D, W>(p, pb, r, kvh, G, cg, sq, (u32)__builtin_ctzll(todo), cps);
+            merge_slice<D, W>(p, pb, n_split, r, kvh, G, cg, sq, (u32)__builtin_ctzll(todo), cps);
         return;
     }
     if (tid == 0)
@@ -1679,14 +1739,15 @@ __device__ __attribute__((always_inline)) inline void decode_ring_body(const Dec
         __hip_atomic_store(arrive, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     if (!closer) return;
     /* (m, l) pairs of the partials: cg * n_split <= 2048 (ring memory) */
-    split_merge_regs<D, CGT, NT>(p, pb, kvh, r, G, cg, sq, (float2 *)&s_ring[0][0]);
+    static_assert(CGT * D / 4 <= NT, "a merging thread per column");
+    split_merge_regs<D, NT>(p, pb, ml_g, n_split, kvh, r, G, cg, sq, (float2 *)&s_ring[0][0]);
 }
 
 /* The kernel: slot indices staged as u32, at most TL_DEC_MAX_CHUNK keys per
  * workgroup when a slot table is staged. */
 template <int D, int G, bool ROPE, bool Q8, bool MF>
 __global__ __launch_bounds__(64 * TL_RING_WAVES) void attn_decode_ring_kernel(const DecParams p) {
-    decode_ring_body<D, G, ROPE, Q8, MF, false>(p);
+    decode_ring_body<D, G, ROPE, Q8, MF, false, false>(p);
 }
 
 /* The same with slot indices staged as u16 (pools of at most 65536 rows), up
@@ -1694,7 +1755,28 @@ __global__ __launch_bounds__(64 * TL_RING_WAVES) void attn_decode_ring_kernel(co
  * TL_DEC_MAX_CHUNK (f16 cache, matrix-core tile; tl_decode_s16.hip). */
 template <int D, int G, bool ROPE, bool MF>
 __global__ __launch_bounds__(64 * TL_RING_WAVES) void attn_decode_ring_kernel_s16(const DecParams p) {
-    decode_ring_body<D, G, ROPE, false, MF, true>(p);
+    decode_ring_body<D, G, ROPE, false, MF, true, false>(p);
+}
+
+/* Batches of sessions of unequal lengths (DecParams.ragged): an instance of
+ * its own, because the lookup of a workgroup's session and split cost every
+ * other launch 0.3 us (decode at 32/8/64 over 700 keys 8.1 -> 8.4). */
+template <int D, int G, bool ROPE, bool Q8, bool MF>
+__global__ __launch_bounds__(64 * TL_RING_WAVES) void attn_decode_ring_kernel_rag(const DecParams p) {
+    decode_ring_body<D, G, ROPE, Q8, MF, false, true>(p);
+}
+
+/* Tiles on the matrix cores for launches of one row per group, where measured
+ * faster (8 kv-heads, 1K and 32K keys, gqa 1-8): the f16 cache at head_dim 64
+ * and 128 from gqa 2 (gqa 8: 16.3 vs 38.3 us at 32K keys; gqa 1 even); the
+ * Q8_0 cache at head_dim 64 from gqa 2 and at 128 from gqa 4 (gqa 8: 26.9 vs
+ * 57.9 us; with two ring tiles per softmax chain the matrix tile takes 24.3
+ * vs 24.65 us at gqa 4 and 8 kv-heads, 16.4 vs 17.9 at 4 kv-heads; gqa 1
+ * stays on the vector tile: 17.7 vs 25.9 us).  At head_dim 256 (8-key tiles,
+ * half of each 16-key block padding) the vector tile is faster (gqa 2: 13.1
+ * vs 13.4 us per launch). */
+constexpr bool tl_decode_matrix_tile(int D, int G, bool q8) {
+    return D == 64 ? G >= 2 : D == 128 ? G >= (q8 ? 4 : 2) : false;
 }
 
 /* One decode kernel instance: entry point, K (or V) bytes per wave tile and
@@ -1710,4 +1792,7 @@ struct DecKernel {
 DecKernel tl_pick_decode_q8(int D, int G, bool rope, bool mf);
 /* the u16-slot instances (f16 cache, matrix-core tile; tl_decode_s16.hip) */
 DecKernel tl_pick_decode_s16(int D, int G, bool rope);
-
+/* the unequal-length instances, tile as tl_decode_matrix_tile (tl_decode_rag.hip,
+ * tl_decode_rag_q8.hip) */
+DecKernel tl_pick_decode_rag(int D, int G, bool rope);
+DecKernel tl_pick_decode_rag_q8(int D, int G, bool rope);

@@ -65,8 +65,15 @@ struct DecParams {
     RopeCfg rope;            /* applied to q and to new K rows */
     uint32_t *counters;      /* merge counters (TL_MERGE_CNT_WORDS, layout below);
                                 NULL = partials are merged by attn_merge_kernel */
-    uint32_t dist;           /* 1: every split merges its own slice of the output */
+    uint32_t dist;           /* n > 0: in groups of at least n splits every split merges its
+                                own slice of the output */
     uint32_t polls;          /* most polls per bounded wait of the split merge */
+    /* sessions of unequal lengths: each has as many splits of `chunk` keys as
+     * it fills; session i's workgroups are [wg0[i], wg0[i + 1]), n_kv groups of
+     * equal split counts (n_split is the largest).  0: every group n_split */
+    uint32_t ragged;
+    uint32_t wg0[TL_MAX_BATCH_SEQ + 1];
+    uint32_t dist_groups;    /* groups whose splits merge slices (dist) */
     uint32_t rows_per_wg;    /* matrix-core tile: batch rows per workgroup group (their
                                 heads side by side as the MFMA columns); 0 or 1: one */
 };
@@ -84,6 +91,17 @@ struct DecParams {
 #define TL_MERGE_MAX_GROUPS 4096
 #define TL_MERGE_PAD 32
 #define TL_MERGE_MAX_SPLIT_DIST 64
+/* A group's last workgroup merges all of it, unless there is much for one CU to
+ * read and enough splits to share it: then every split merges a slice, at one
+ * more round trip each.  A slice takes its workgroup's 8 waves one float4 each,
+ * so 16 or fewer per split are two rounds.  us per launch, last workgroup /
+ * slices, at head_dim 128 (columns = rows x heads of a group): 16 columns x 32
+ * splits (256 KB of partials) 16.8 / 16.3, 8 x 32 (128 KB) 15.0 / 14.7, 7 x 64
+ * 16.9 / 15.0; but 4 x 32 (64 KB) 28.1 / 28.3, 14 x 21 (147 KB, three rounds)
+ * 14.6 / 15.3, 7 x 16 10.1 / 11.3. */
+#define TL_MERGE_MIN_SPLIT_DIST 24
+#define TL_MERGE_MIN_BYTES_DIST (72u << 10)
+#define TL_MERGE_SLICE_MAX 16
 #define TL_MERGE_TAGS (TL_MERGE_MAX_GROUPS * TL_MERGE_PAD)
 #define TL_MERGE_LAUNCHES (TL_MERGE_TAGS + TL_MERGE_MAX_SPLIT_DIST * TL_MERGE_MAX_GROUPS)
 /* groups of the current launch whose closer has run (dist merge): the last
