@@ -16,6 +16,7 @@ typedef float floatx16_t __attribute__((ext_vector_type(16)));
 template <int D>
 constexpr int pf_keys() { return D <= 128 ? 64 : 32; }
 
+#define PF_AHEAD 4   /* K operands read ahead of the MFMA that takes them */
 #define PF_WPE(D) (D == 256 ? 1 : 2)   /* waves per SIMD: 512 or 256 registers */
 #define TL_PF_VPAD 32      /* V row padding in halves: a transpose read's 16-lane
                               group hits 4 rows x 32 B at row steps of 16 (or 48)
@@ -347,17 +348,25 @@ __global__ __attribute__((amdgpu_flat_work_group_size(64 * W, 64 * W), amdgpu_wa
          * 32 kb + 8(r/4) + 4h + r%4 of query lr */
         floatx16_t sacc[KB];
 #pragma unroll
-        for (int kb = 0; kb < KB; kb++) {
-            const int krow = 32 * kb + lr;
-            sacc[kb] = __builtin_amdgcn_mfma_f32_32x32x16_f16(
-                h8_from_u4(sk[krow * CPR + (h ^ (krow % CPR))]), qop[0], bias, 0, 0, 0);
+        for (int s = 0; s < KS; s++)
 #pragma unroll
-            for (int s = 1; s < KS; s++) {
-                const int c = 2 * s + h;
+            for (int kb = 0; kb < KB; kb++) {
+                const int krow = 32 * kb + lr, c = 2 * s + h;
                 const half8_t a = h8_from_u4(sk[krow * CPR + (c ^ (krow % CPR))]);
-                sacc[kb] = __builtin_amdgcn_mfma_f32_32x32x16_f16(a, qop[s], sacc[kb], 0, 0, 0);
+                sacc[kb] = __builtin_amdgcn_mfma_f32_32x32x16_f16(a, qop[s], s ? sacc[kb] : bias, 0, 0, 0);
             }
+        /* PF_AHEAD operand reads in flight ahead of each MFMA, the key blocks'
+         * chains in turn: left alone, the scheduler waits out every read
+         * before its MFMA (512 rows, us: from position 0 at 32/8/128 23.6 ->
+         * 22.5, 28/4/128 23.4 -> 22.4; over 32K keys at 32/8/64 175 -> 171, at
+         * 32/8/128 287 -> 283; 6 ahead is slower again on short launches) */
+        __builtin_amdgcn_sched_group_barrier(0x100, PF_AHEAD, 0);
+#pragma unroll
+        for (int i = 0; i < KB * KS - PF_AHEAD; i++) {
+            __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+            __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
         }
+        __builtin_amdgcn_sched_group_barrier(0x008, PF_AHEAD, 0);
 
         /* mask (only tiles that cross a boundary; visible keys of this lane's
          * row are [klo, khi)) + online softmax.  The reference mu is raised
