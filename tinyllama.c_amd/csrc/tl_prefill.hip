@@ -216,7 +216,9 @@ bool tl_use_prefill(const LayerView &L, const tl_attn_args *a) {
     return a->n > TL_DEC_FOLD_MAX_ROWS || (u64)a->n * vis > work;
 }
 
-static u32 task_blocks(u32 n, u32 G, u32 W) { return (G * ((n + 31) / 32) + W - 1) / W; }
+/* workgroups of W tasks per kv-head; GN = tasks of a 32-row block */
+static u32 task_blocks(u32 n, u32 GN, u32 W) { return (GN * ((n + 31) / 32) + W - 1) / W; }
+static u32 tasks_per_block(u32 D, u32 G) { return D == 256 ? G * pf_parts<256>() : G; }
 
 /* Waves per workgroup (W) and key splits of a launch, by a cost in us: the
  * tiles of one workgroup's share of the keys, plus, with splits, the merge
@@ -225,32 +227,33 @@ static u32 task_blocks(u32 n, u32 G, u32 W) { return (G * ((n + 31) / 32) + W - 
  * at 28/4/128 over 16K keys: 4 splits 148 us, 5 splits 221).
  * One tile (64 keys; 32 at head_dim 256) of a workgroup takes 1.70 us with 8
  * waves and 1.55 with 4 at head_dim 128 (long runs, one workgroup per CU),
- * 1.18 / 0.94 at 64, 1.75 with 4 at 256, ~2.1 over a Q8_0 cache, where the
+ * 1.18 / 0.94 at 64, 1.39 / 1.50 at 256, ~2.1 over a Q8_0 cache, where the
  * dequantization is shared by the workgroup's threads.  So 8 waves read and
  * stage each key for twice the rows at nearly the same speed and win where
  * they fill the chip; 4 waves start ~3 us sooner (half the rows to append and
- * stage) and win below that.  Measured, W = 8 / 4, best split counts (us): 512
+ * stage; not at 256, where two waves share a row block and head) and win below
+ * that.  Measured, W = 8 / 4, best split counts (us): 512
  * rows from position 0 at 32/8/128 27.1 / 23.3, 333 at 28/4/128 23.4 / 18.3,
  * 512 at 32/8/64 20.5 / 16.0; 333 rows over 1K keys at 32/8/64 21.4 / 19.7;
  * 100 over 2K 18.7 / 16.6; 512 rows over 4.6K keys at 32/8/128 58.9 / 62.2,
  * at 32/8/64 39.3 / 40.0; 70 rows over 20K at 28/4/128 52.3 / 53.7. */
 static void plan(const LayerView &L, const tl_attn_args *a, u32 G, u32 cus, u32 &W, u32 &ns) {
-    const u32 D = L.head_dim, bn = D <= 128 ? 64 : 32;
+    const u32 D = L.head_dim, bn = D <= 128 ? 64 : 32, GN = tasks_per_block(D, G);
     const float part_us = (float)a->n * a->n_head * D * 4.f * 2.f / 5e6f;   /* per split */
     float best = 0.f;
     W = 0;
-    for (u32 w = D == 256 ? 4 : 8; w >= 4; w -= 4) {
-        const float tile = (L.q8 ? 2.1f : D == 64 ? (w == 8 ? 1.18f : 0.94f)
-                                 : D == 128 ? (w == 8 ? 1.70f : 1.55f) : 1.75f);
-        const u32 base = task_blocks(a->n, G, w) * L.n_kv_head;
+    for (u32 w = 8; w >= 4; w -= 4) {
+        const float tile = L.q8 ? 2.1f : D == 64 ? (w == 8 ? 1.18f : 0.94f)
+                                       : D == 128 ? (w == 8 ? 1.70f : 1.55f) : (w == 8 ? 1.39f : 1.5f);
+        const u32 base = task_blocks(a->n, GN, w) * L.n_kv_head;
         if (base > cus && W) break;
-        const u32 rows = ((w - 1) / G + 1) * 32;
+        const u32 rows = ((w - 1) / GN + 1) * 32;
         u32 span = a->pos + a->n;              /* most keys any workgroup sees */
         if (a->window && span > a->window + rows) span = a->window + rows;
         const u32 most = base < cus ? cus / base : 1u;
         for (u32 k = 1; k <= most; k++) {
             const u32 tiles = ((span + k - 1) / k + bn - 1) / bn;
-            const float t = tiles * tile + (w == 8 ? 3.f : 0.f) + (k > 1 ? 5.f + k * part_us : 0.f);
+            const float t = tiles * tile + (w == 8 && D <= 128 ? 3.f : 0.f) + (k > 1 ? 5.f + k * part_us : 0.f);
             if (!W || t < best) {
                 best = t;
                 W = w;
@@ -302,7 +305,7 @@ int tl_launch_prefill(const LayerView &L, const tl_attn_args *a, const RopeCfg &
     }
     u32 W, ns;
     plan(L, a, G, (u32)cus, W, ns);
-    const u32 base = task_blocks(a->n, G, W) * L.n_kv_head;
+    const u32 base = task_blocks(a->n, tasks_per_block(D, G), W) * L.n_kv_head;
     if (const u32 t = tl_tune(TL_TUNE_PREFILL_SPLITS)) ns = t;
     if (const size_t fixed = tl_workspace_fixed_acc()) {
         /* no-allocation call: as many key splits as the fixed region holds */

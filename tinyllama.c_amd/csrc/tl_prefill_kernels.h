@@ -15,9 +15,16 @@ typedef float floatx16_t __attribute__((ext_vector_type(16)));
 /* keys per LDS tile */
 template <int D>
 constexpr int pf_keys() { return D <= 128 ? 64 : 32; }
+/* waves that share a (row block, q-head): at head_dim 256 two, each with all of
+ * S and half of O's dims, so a wave fits 256 registers and a SIMD holds two.
+ * One wave with all of O took 446, half of them accumulation registers that it
+ * moved on every tile, alone on its SIMD: 1.97 us per 32-key tile of a 4-task
+ * workgroup, 1.39 this way (512 rows over 8.7K keys at 8/4/256: 89 -> 77 us),
+ * though S is computed twice */
+template <int D>
+constexpr int pf_parts() { return D <= 128 ? 1 : 2; }
 
 #define PF_AHEAD 4   /* K operands read ahead of the MFMA that takes them */
-#define PF_WPE(D) (D == 256 ? 1 : 2)   /* waves per SIMD: 512 or 256 registers */
 #define TL_PF_VPAD 32      /* V row padding in halves: a transpose read's 16-lane
                               group hits 4 rows x 32 B at row steps of 16 (or 48)
                               banks, and the group 32 B to its right fills the
@@ -49,12 +56,13 @@ TL_DEV uint2 ld_tr16(const _Float16 *lds_ptr) {
 }
 
 template <int D, int W, bool Q8>
-__global__ __attribute__((amdgpu_flat_work_group_size(64 * W, 64 * W), amdgpu_waves_per_eu(PF_WPE(D)))) void attn_prefill_kernel(const PrefParams p) {
+__global__ __attribute__((amdgpu_flat_work_group_size(64 * W, 64 * W), amdgpu_waves_per_eu(2))) void attn_prefill_kernel(const PrefParams p) {
     constexpr int BN = pf_keys<D>();
     constexpr int T = 64 * W;
     constexpr int CPR = D / 8;           /* 16-byte chunks per row */
     constexpr int KS = D / 16;           /* k-steps of the QK MFMA */
-    constexpr int DB = D / 32;           /* 32-row d-blocks of O^T */
+    constexpr int NP = pf_parts<D>();
+    constexpr int DB = D / 32 / NP;      /* 32-row d-blocks of O^T of a wave */
     constexpr int KB = BN / 32;          /* 32-key blocks of S^T per tile */
     constexpr int UNITS = BN * CPR;      /* 16-byte units per K (or V) tile */
     constexpr int UPT = (UNITS + T - 1) / T;
@@ -120,10 +128,12 @@ __global__ __attribute__((amdgpu_flat_work_group_size(64 * W, 64 * W), amdgpu_wa
     const u32 x = blockIdx.x % nx, tblk = gridDim.x / nx - 1 - blockIdx.x / nx;
     const u32 kvh = x / p.n_split, split = x % p.n_split;
 
-    /* task t of a kv-head = (32-row block t / G, q-head t % G); wave w of the
-     * workgroup has task tblk * W + w, or none past the last */
-    const u32 G = p.gqa, t0 = tblk * W, qb = (t0 + wave) / G;
-    const u32 hq = kvh * G + (t0 + wave) % G;
+    /* task t of a kv-head = (32-row block t / GN, q-head (t % GN) / NP, part of
+     * O's dims t % NP), GN = gqa * NP; wave w of the workgroup has task
+     * tblk * W + w, or none past the last */
+    const u32 GN = p.gqa * NP, t0 = tblk * W, qb = (t0 + wave) / GN;
+    const u32 hq = kvh * p.gqa + (t0 + wave) % GN / NP;
+    const u32 dpart = NP == 1 ? 0u : (t0 + wave) % NP * (D / NP);   /* first dim of the wave's O */
     const bool busy = qb * 32 < p.n;
     const u32 my_q = qb * 32 + lr;                   /* lane's query row */
     const bool row_ok = my_q < p.n;
@@ -133,8 +143,8 @@ __global__ __attribute__((amdgpu_flat_work_group_size(64 * W, 64 * W), amdgpu_wa
     const u32 wq1 = p.pos + min(qb * 32 + 31, p.n - 1);
 
     /* key range of the workgroup's rows, then of this split */
-    const u32 wg_last = p.pos + min(((t0 + W - 1) / G + 1) * 32, p.n);
-    const u32 first_pos = p.pos + t0 / G * 32;
+    const u32 wg_last = p.pos + min(((t0 + W - 1) / GN + 1) * 32, p.n);
+    const u32 first_pos = p.pos + t0 / GN * 32;
     const u32 wg_first = (p.window && first_pos + 1 > p.window) ? first_pos + 1 - p.window : 0;
     const u32 span = wg_last - wg_first;
     u32 chunk = (span + p.n_split - 1) / p.n_split;
@@ -311,7 +321,7 @@ __global__ __attribute__((amdgpu_flat_work_group_size(64 * W, 64 * W), amdgpu_wa
     /* transpose-read coordinates of this lane (16-lane group gi, lane i) */
     const int gi = lane >> 4, li = lane & 15;
     const int tr_row = li >> 2;                       /* + 4h (+8) + 16 kb4 */
-    const int tr_col = 16 * (gi & 1) + 4 * (li & 3);  /* + 32 b */
+    const int tr_col = 16 * (gi & 1) + 4 * (li & 3) + (int)dpart;  /* + 32 b */
 
     /* the workgroup reads batch rows: all their units must be in the cache
      * before its first load (the writers published at their start) */
@@ -475,9 +485,9 @@ __global__ __attribute__((amdgpu_flat_work_group_size(64 * W, 64 * W), amdgpu_wa
         __hip_atomic_fetch_add(p.ctr, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     }
     if (!row_ok) return;
-    /* o[b][r] = O^T[d = 32b + 8(r/4) + 4h + r%4][row lr] */
+    /* o[b][r] = O^T[d = dpart + 32b + 8(r/4) + 4h + r%4][row lr] */
     if (p.n_split == 1) {
-        float *dst = p.dst + (u64)my_q * p.q_stride + (u64)hq * D;
+        float *dst = p.dst + (u64)my_q * p.q_stride + (u64)hq * D + dpart;
         const float inv = 1.0f / lsum;
 #pragma unroll
         for (int b = 0; b < DB; b++)
@@ -485,12 +495,12 @@ __global__ __attribute__((amdgpu_flat_work_group_size(64 * W, 64 * W), amdgpu_wa
             for (int r = 0; r < 16; r++) dst[32 * b + 8 * (r / 4) + 4 * h + (r % 4)] = o[b][r] * inv;
     } else {
         const u64 pi = ((u64)my_q * p.n_head + hq) * p.n_split + split;
-        float *acc = p.ws_acc + pi * D;
+        float *acc = p.ws_acc + pi * D + dpart;
 #pragma unroll
         for (int b = 0; b < DB; b++)
 #pragma unroll
             for (int r = 0; r < 16; r++) acc[32 * b + 8 * (r / 4) + 4 * h + (r % 4)] = o[b][r];
-        if (h == 0) p.ws_ml[pi] = make_float2(m, lsum);
+        if (h == 0 && dpart == 0) p.ws_ml[pi] = make_float2(m, lsum);
     }
 }
 
@@ -503,7 +513,8 @@ __global__ __attribute__((amdgpu_flat_work_group_size(64 * W, 64 * W), amdgpu_wa
                       : W == 4 ? (const void *)attn_prefill_kernel<64, 4, Q8> : nullptr;     \
         case 128: return W == 8 ? (const void *)attn_prefill_kernel<128, 8, Q8>              \
                        : W == 4 ? (const void *)attn_prefill_kernel<128, 4, Q8> : nullptr;   \
-        case 256: return W == 4 ? (const void *)attn_prefill_kernel<256, 4, Q8> : nullptr;   \
+        case 256: return W == 8 ? (const void *)attn_prefill_kernel<256, 8, Q8>              \
+                       : W == 4 ? (const void *)attn_prefill_kernel<256, 4, Q8> : nullptr;   \
         default: return nullptr;                                                             \
         }                                                                                    \
     }
