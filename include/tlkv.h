@@ -170,7 +170,8 @@ int tl_kv_copy_between(const tl_kv_layer *dst_layers, const tl_kv_layer *src_lay
  * reference runs OP_ROPE on Q and K, cpu_op.c:637-700, then OP_ATTN,
  * cpu_op.c:964-1064).  Same results as tl_rope(q rows at pos..), tl_rope(k
  * rows at pos..) then tl_attn, bit for bit, in one launch for decode batches
- * (two for prefill batches: append+RoPE, then attention).  q and k are read,
+ * (two for prefill batches: rotation and append, then attention; dst holds
+ * the rotated q between them).  q and k are read,
  * not rotated in place. */
 int tl_attn_rope(const tl_kv_layer *L, const tl_attn_args *a, const tl_rope_params *rope,
                  void *stream);

@@ -197,23 +197,33 @@ bool tl_prefill_supported(const LayerView &L, const tl_attn_args *a) {
     return (L.head_dim == 64 || L.head_dim == 128 || L.head_dim == 256) && G >= 1 && G <= 8;
 }
 
-/* The prefill kernel for batches of at least TL_PREFILL_MIN_ROWS rows whose
- * rows x visible keys exceed TL_PREFILL_MIN_WORK (or of more than
- * TL_DEC_FOLD_MAX_ROWS rows); smaller ones run on the decode kernel, whose
- * matrix tile folds the rows into its columns.  Measured (f16, 8 or 4
- * kv-heads, head_dim 64-256, us per launch, decode vs prefill kernel): 64
- * rows at 1K keys 16.0 vs 25.6, at 2K 21.0 vs 27.9; 32 rows at 4K 21.4 vs
- * 26.3; 16 rows at 8K 19.5 vs 26.2, 24 rows 27.4 vs 27.0; 32 rows at 8K
- * 46.9 vs 28.0; 16 rows at 16K 49.3 vs 31.8.  The Q8_0 cache's decode tile
- * is dearer per key: 32 rows at 4K 27.1 vs 29.1, 48 rows 56.0 vs 32.4; 16
- * rows at 8K 28.4 vs 30.4, 24 rows 37.5 vs 32.2. */
+/* The prefill kernel for batches of more than TL_DEC_FOLD_MAX_ROWS rows, and for
+ * those of at least TL_PREFILL_MIN_ROWS whose rows x visible keys x heads x
+ * head_dim exceed a bound; smaller ones run on the decode kernel, whose matrix
+ * tile folds the rows into its columns; a quantized key is dearer there.  The
+ * bound is the same with RoPE, so that a fused call takes the kernel, and gives
+ * the bits, of the rotation and the plain call; with it the prefill side would
+ * win earlier, because the decode side needs a rotating append launch first
+ * (28/4/128 NEOX, 32 rows over 500 keys 18.7 / 17.5).  Measured, us per OP_ATTN,
+ * decode / prefill kernel (32/8/128 unless said): f16, 17 rows over 4K keys 19.9
+ * / 20.2, 8K 26.9 / 22.6; 32 rows 2K 17.7 / 19.6, 4K 23.3 / 22.5; 64 rows 1K
+ * 17.6 / 19.5, 2K 23.2 / 22.5, 4K 33.6 / 24.5; 32/8/64, 32 rows 4K 15.1 / 17.1,
+ * 8K 20.3 / 20.5, 16K 29.4 / 23.7; 8/4/256, 32 rows 2K 21.5 / 22.7, 4K 29.9 /
+ * 26.5.  Q8_0, 32 rows 1K 17.1 / 21.4, 2K 22.9 / 23.2, 4K 31.0 / 27.0; 8/4/256
+ * 2K 24.8 / 24.8. */
+static u64 prefill_min_work(const LayerView &L) {
+    const bool wide = L.head_dim == 256;
+    if (L.q8) return wide ? 180000000u : 250000000u;
+    return wide ? 200000000u : 400000000u;
+}
+
 bool tl_use_prefill(const LayerView &L, const tl_attn_args *a) {
     if (a->n < TL_PREFILL_MIN_ROWS || !tl_prefill_supported(L, a)) return false;
     if (tl_tune(TL_TUNE_NO_PREFILL) == 2) return true;
     const u64 keys = (u64)a->pos + a->n;
     const u64 vis = (a->window && keys > a->window) ? a->window : keys;
-    const u64 work = L.q8 ? TL_PREFILL_MIN_WORK_Q8 : TL_PREFILL_MIN_WORK;
-    return a->n > TL_DEC_FOLD_MAX_ROWS || (u64)a->n * vis > work;
+    return a->n > TL_DEC_FOLD_MAX_ROWS ||
+           (u64)a->n * vis * a->n_head * L.head_dim > prefill_min_work(L);
 }
 
 /* workgroups of W tasks per kv-head; GN = tasks of a 32-row block */
