@@ -532,6 +532,23 @@ def test_prefill_task_packing(T, case, splits):
     assert np.abs(out - o32).max() < TOL
 
 
+# windows that reach past the first key hide nothing, up to "no limit" as the
+# largest number and the last ones whose sum with a position passes 2^32
+@pytest.mark.parametrize("window", [2 ** 32 - 1, 2 ** 32 - 600, 2 ** 31, 900])
+@pytest.mark.parametrize("case", [(8, 2, 128, 700, 130), (4, 4, 64, 300, 500), (2, 1, 256, 830, 65)])
+def test_prefill_window_wider_than_context(T, case, window):
+    import tlkv
+    n_head, n_kv, hd, pos, n = case
+    outs = []
+    with tlkv.tuning(tlkv.TUNE_NO_PREFILL, 2):
+        for w in (0, window):
+            out, o16, _, _, _ = _run_attn(T, n_head, n_kv, hd, pos + n, pos, n, w, None, seed=n)
+            assert np.abs(out - o16).max() < TOL, w
+            outs.append(out)
+    # the same plan and the same keys: masked tiles add nothing to a row's bits
+    assert np.array_equal(outs[0].view(np.uint32), outs[1].view(np.uint32))
+
+
 def test_prefill_split_invariance(T):
     outs = []
     import tlkv

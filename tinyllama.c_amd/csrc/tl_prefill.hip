@@ -259,7 +259,7 @@ static void plan(const LayerView &L, const tl_attn_args *a, u32 G, u32 cus, u32 
         if (base > cus && W) break;
         const u32 rows = ((w - 1) / GN + 1) * 32;
         u32 span = a->pos + a->n;              /* most keys any workgroup sees */
-        if (a->window && span > a->window + rows) span = a->window + rows;
+        if (a->window && span > (u64)a->window + rows) span = a->window + rows;
         const u32 most = base < cus ? cus / base : 1u;
         for (u32 k = 1; k <= most; k++) {
             const u32 tiles = ((span + k - 1) / k + bn - 1) / bn;
