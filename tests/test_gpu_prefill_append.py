@@ -101,7 +101,16 @@ def _run(T, case, mode):
     return res
 
 
-@pytest.mark.parametrize("case", CASES, ids=lambda c: f"h{c[0]}-kv{c[1]}-d{c[2]}-p{c[4]}-n{c[5]}")
+# more 16-row units than a workgroup of the launch has threads (4 waves: 4096
+# rows, 8 waves: 8192): every one has to be in the cache before it is read
+LONG_CASES = [
+    (4, 2, 128, 4112, 0, 4112, 64, 0, False, None),       # 4 waves, 257 units
+    (2, 1, 256, 4300, 150, 4112, 64, 0, True, None),      # 4 waves, head_dim 256
+    (4, 1, 128, 8208, 0, 8208, 64, 0, False, None),       # 8 waves, 513 units
+]
+
+
+@pytest.mark.parametrize("case", CASES + LONG_CASES, ids=lambda c: f"h{c[0]}-kv{c[1]}-d{c[2]}-p{c[4]}-n{c[5]}")
 def test_fused_append_equals_separate(T, case):
     base = _run(T, case, "separate")
     assert np.abs(base["out"] - base["ref"]).max() < TOL

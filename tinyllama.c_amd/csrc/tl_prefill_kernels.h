@@ -258,15 +258,22 @@ __global__ __attribute__((amdgpu_flat_work_group_size(64 * W, 64 * W), amdgpu_wa
      * stores were written through before their flags were set. */
     auto await_batch = [&]() __attribute__((always_inline)) {
         const u32 need = (wg_last - p.pos + TL_PF_ROWS - 1) / TL_PF_ROWS;
-        if ((u32)tid < need) {
-            const u32 *fl = p.flags + kvh * n_units + (u32)tid;
+        auto wait_unit = [&](u32 u) __attribute__((always_inline)) {
+            const u32 *fl = p.flags + kvh * n_units + u;
             bool ok = false;
             for (u32 it = 0; it < p.polls && !ok; it++) {
                 if (it) __builtin_amdgcn_s_sleep(4);
                 ok = __hip_atomic_load(fl, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == epoch;
             }
             if (!ok) s_direct = 1u;
-        }
+            return ok;
+        };
+        /* thread i: unit i, and with more units than threads i + T, ...
+         * (apart: one loop over all of them costs each short launch 0.8 us) */
+        bool ok = true;
+        if ((u32)tid < need) ok = wait_unit((u32)tid);
+        if (need > (u32)T)
+            for (u32 u = (u32)tid + T; ok && u < need; u += T) ok = wait_unit(u);
         __syncthreads();
         if (s_direct) {
             for (u32 b = 0; b < need; b++) write_unit(kvh, b * TL_PF_ROWS);
