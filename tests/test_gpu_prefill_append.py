@@ -120,3 +120,33 @@ def test_fused_append_equals_separate(T, case):
         assert np.array_equal(got["v"], base["v"]), f"{mode}: V cache differs"
         assert np.array_equal(got["out"].view(np.uint32), base["out"].view(np.uint32)), mode
         assert np.abs(got["out"] - got["ref"]).max() < TOL, mode
+
+
+@pytest.mark.parametrize("shape", [(32, 8, 128, 3072), (12, 4, 64, 6000), (8, 4, 256, 4128)])
+def test_long_batch_does_not_wait_for_later_workgroups(T, shape):
+    """More workgroups than the chip runs at once: the append must not be
+    fused, or workgroups wait, up to the bound, for rows that later ones write
+    (measured: 10 times the separate append's time; the bound here is 3)."""
+    import tlkv
+    nh, nkv, hd, n = shape
+    lib = tlkv.lib()
+    g = T.Generator(device="cuda")
+    g.manual_seed(n)
+    q, k, v = (T.randn((n, h * hd), generator=g, device="cuda") for h in (nh, nkv, nkv))
+    L, times, outs = tlkv.Layer(n, nkv, hd), [], []
+    for separate in (1, 0):
+        out = T.zeros_like(q)
+        a = tlkv.attn_args(q, k, v, out, None, 0, n, nh, hd, nkv, 64, O.scale_of(hd))
+        with tlkv.tuning(tlkv.TUNE_PREFILL_SEPARATE_APPEND, separate):
+            t = []
+            for _ in range(6):
+                e0, e1 = (T.cuda.Event(enable_timing=True) for _ in range(2))
+                e0.record()
+                tlkv.check(lib.tl_attn(L.desc, a, tlkv.stream_handle()))
+                e1.record()
+                T.cuda.synchronize()
+                t.append(e0.elapsed_time(e1))
+        times.append(min(t))
+        outs.append(out)
+    assert T.equal(outs[0], outs[1])
+    assert times[1] < 3 * times[0] + 0.05, times

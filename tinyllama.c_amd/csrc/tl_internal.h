@@ -203,7 +203,8 @@ int tl_launch_merge(const DecParams &p, uint32_t n_rows_total, uint32_t head_dim
 bool tl_prefill_supported(const LayerView &L, const tl_attn_args *a);
 /* the batch runs on the prefill kernel (else on the decode kernel) */
 bool tl_use_prefill(const LayerView &L, const tl_attn_args *a);
-/* append: the launch writes the batch rows itself (f16 cache); with RoPE the
- * rotating pre-launch writes them, into either cache */
+/* append: the launch writes the batch rows itself (f16 cache), or, where its
+ * grid is too large for that and `own` is given, own's append launch does; with
+ * RoPE the rotating pre-launch writes them, into either cache */
 int tl_launch_prefill(const LayerView &L, const tl_attn_args *a, const RopeCfg &rope,
-                      hipStream_t st, bool append = false);
+                      hipStream_t st, bool append = false, const AppendParams *own = nullptr);

@@ -683,8 +683,8 @@ static int attn_core(const tl_kv_layer *L, const tl_attn_args *a, bool append,
     const LayerView lv = tl_view(L);
     if (tl_use_prefill(lv, a)) {
         bool fused = false;
+        AppendParams ap;
         if (append) {
-            AppendParams ap;
             memset(&ap, 0, sizeof(ap));
             int rc = fill_seg(ap.seg[0], L, a->k, a->v, a->kv_stride, a->slots, a->pos, a->n);
             if (rc) return rc;
@@ -699,7 +699,7 @@ static int attn_core(const tl_kv_layer *L, const tl_attn_args *a, bool append,
                 if (rc) return rc;
             }
         }
-        return tl_launch_prefill(lv, a, rope, st, fused);
+        return tl_launch_prefill(lv, a, rope, st, fused, &ap);
     }
     DecParams p;
     memset(&p, 0, sizeof(p));

@@ -275,7 +275,7 @@ static void plan(const LayerView &L, const tl_attn_args *a, u32 G, u32 cus, u32 
 }
 
 int tl_launch_prefill(const LayerView &L, const tl_attn_args *a, const RopeCfg &rope,
-                      hipStream_t st, bool append) {
+                      hipStream_t st, bool append, const AppendParams *own) {
     const bool rope_on = rope.rdim != 0;
     if (append && L.q8 && !rope_on)
         return tl_fail(TL_EINVAL, "prefill: no fused append into a Q8_0 cache");
@@ -324,6 +324,20 @@ int tl_launch_prefill(const LayerView &L, const tl_attn_args *a, const RopeCfg &
         if (ns < 1) ns = 1;
     }
     p.n_split = ns;
+    const u32 blocks = base * ns;
+    if (append && own && blocks > (u32)cus) {
+        /* workgroups of the fused append wait for units that other workgroups
+         * write, so all of them have to run at once: one per CU is sure to.
+         * With more, a writer may not start before a waiter ends, every such
+         * wait runs into its bound and the waiter writes all the rows itself
+         * (us per OP_ATTN from position 0, fused / separate: 3072 rows at
+         * 32/8/128, 384 workgroups, 1147 / 113; 4096 rows at 32/8/64, 512
+         * workgroups, 1264 / 113; where all run at once fusing is the faster:
+         * 4096 rows at 8/8/128 86 / 88, 3072 rows at 4/1/128 39.8 / 43.4) */
+        const int rc = tl_launch_append(*own, 1, st);
+        if (rc) return rc;
+        append = false;
+    }
     const size_t units = (size_t)L.n_kv_head * ((a->n + TL_PF_ROWS - 1) / TL_PF_ROWS);
     if (ns > 1 || append) {
         TlWorkspace *w;
@@ -347,7 +361,6 @@ int tl_launch_prefill(const LayerView &L, const tl_attn_args *a, const RopeCfg &
             p.polls = polls ? polls - 1 : 4096;
         }
     }
-    const u32 blocks = base * ns;
     const void *fn = L.q8 ? tl_prefill_fn_q8((int)D, (int)W) : tl_prefill_fn((int)D, (int)W);
     if (!fn) return tl_fail(TL_EINVAL, "prefill: head_dim %u gqa %u", D, G);
     if (rope_on) {
