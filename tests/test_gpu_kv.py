@@ -532,6 +532,34 @@ def test_prefill_task_packing(T, case, splits):
     assert np.abs(out - o32).max() < TOL
 
 
+@pytest.mark.parametrize("case", [(1, 1, 64, 12000, 65), (1, 1, 64, 12000, 200)])
+def test_prefill_plan_counts_the_merge(T, case):
+    """Few heads and many keys: the planned split count is no slower than a
+    sixth or a third of as many splits as there are CUs (measured 1.0 times the
+    best of them; 1.75 and 1.28 when the merge of a split cost nothing)."""
+    import tlkv
+    n_head, n_kv, hd, pos, n = case
+    g = T.Generator(device="cuda")
+    g.manual_seed(n)
+    L = tlkv.Layer(pos + n, n_kv, hd)
+    q, k, v = (T.randn((n, h * hd), generator=g, device="cuda") for h in (n_head, n_kv, n_kv))
+    a = tlkv.attn_args(q, k, v, T.zeros_like(q), None, pos, n, n_head, hd, n_kv, 0, O.scale_of(hd))
+    times = []
+    for splits in (0, 32, 48):
+        with tlkv.tuning(tlkv.TUNE_PREFILL_SPLITS, splits):
+            t = []
+            for _ in range(8):
+                e0, e1 = (T.cuda.Event(enable_timing=True) for _ in range(2))
+                e0.record()
+                for _ in range(20):
+                    tlkv.check(tlkv.lib().tl_attn(L.desc, a, tlkv.stream_handle()))
+                e1.record()
+                T.cuda.synchronize()
+                t.append(e0.elapsed_time(e1))
+        times.append(min(t))
+    assert times[0] < 1.2 * min(times[1:]), times
+
+
 # windows that reach past the first key hide nothing, up to "no limit" as the
 # largest number and the last ones whose sum with a position passes 2^32
 @pytest.mark.parametrize("window", [2 ** 32 - 1, 2 ** 32 - 600, 2 ** 31, 900])

@@ -230,31 +230,49 @@ bool tl_use_prefill(const LayerView &L, const tl_attn_args *a) {
 static u32 task_blocks(u32 n, u32 GN, u32 W) { return (GN * ((n + 31) / 32) + W - 1) / W; }
 static u32 tasks_per_block(u32 D, u32 G) { return D == 256 ? G * pf_parts<256>() : G; }
 
+/* us per tile (64 keys; 32 at head_dim 256) of a workgroup of w waves: the
+ * slope of long runs with one workgroup per CU (f16 at head_dim 128 1.70 / 1.55
+ * for 8 / 4 waves, at 64 1.1 / 0.9; Q8_0 1.87 / 2.03 and 1.12 / 1.26: there the
+ * workgroup's threads dequantize the tile, so half of them take longer), then
+ * moved to where the plan's choices cost least over 260 shapes (65 to 1024 rows,
+ * 0 to 14K keys, 1 to 32 heads, both caches), each timed at both widths and up
+ * to 16 split counts: the choices are 1.5% from the best ones on average (4.1%
+ * with one Q8_0 cost for all and a merge that costs the same for any count), 7%
+ * for one shape in 20.  At 256 (slopes 1.39 / 1.5, Q8_0 1.63 / 1.9) and for 4
+ * waves over a Q8_0 cache short runs count for more than the slope. */
+static float tile_us(u32 D, u32 w, bool q8) {
+    if (q8) return D == 64 ? (w == 8 ? 1.12f : 1.45f) : D == 128 ? (w == 8 ? 1.90f : 2.10f)
+                                                                 : (w == 8 ? 2.06f : 1.90f);
+    return D == 64 ? (w == 8 ? 1.10f : 0.94f) : D == 128 ? (w == 8 ? 1.70f : 1.55f)
+                                                         : (w == 8 ? 1.39f : 1.19f);
+}
+
 /* Waves per workgroup (W) and key splits of a launch, by a cost in us: the
  * tiles of one workgroup's share of the keys, plus, with splits, the merge
- * launch and the partials' way through memory (~5 TB/s).  At most one
- * workgroup per CU counts: a partial second round doubles the time (512 rows
- * at 28/4/128 over 16K keys: 4 splits 148 us, 5 splits 221).
- * One tile (64 keys; 32 at head_dim 256) of a workgroup takes 1.70 us with 8
- * waves and 1.55 with 4 at head_dim 128 (long runs, one workgroup per CU),
- * 1.18 / 0.94 at 64, 1.39 / 1.50 at 256, ~2.1 over a Q8_0 cache, where the
- * dequantization is shared by the workgroup's threads.  So 8 waves read and
- * stage each key for twice the rows at nearly the same speed and win where
- * they fill the chip; 4 waves start ~3 us sooner (half the rows to append and
- * stage; not at 256, where two waves share a row block and head) and win below
- * that.  Measured, W = 8 / 4, best split counts (us): 512
+ * launch: 3.5 us, 0.11 for each split (a thread folds them in turn; 65 rows at
+ * 1/1/64 over 12K keys: 32 splits 16.4, 189 splits 28.8) and the partials' way
+ * through memory (~6 TB/s; 2048 rows at 12/4/64 from position 0, 8 waves: 1
+ * split 50.4, 2 splits 38.0).  At most one workgroup per CU counts: a partial
+ * second round doubles the time (512 rows at 28/4/128 over 16K keys: 4 splits
+ * 148 us, 5 splits 221).
+ * 8 waves read and stage each key for twice the rows at nearly the same speed
+ * and win where they fill the chip; 4 waves start ~3 us sooner (half the rows
+ * to append and stage) and win below that.  Measured, W = 8 / 4, best split
+ * counts (us): 512
  * rows from position 0 at 32/8/128 27.1 / 23.3, 333 at 28/4/128 23.4 / 18.3,
  * 512 at 32/8/64 20.5 / 16.0; 333 rows over 1K keys at 32/8/64 21.4 / 19.7;
  * 100 over 2K 18.7 / 16.6; 512 rows over 4.6K keys at 32/8/128 58.9 / 62.2,
- * at 32/8/64 39.3 / 40.0; 70 rows over 20K at 28/4/128 52.3 / 53.7. */
+ * at 32/8/64 39.3 / 40.0; 70 rows over 20K at 28/4/128 52.3 / 53.7; Q8_0, 512
+ * rows from position 0 at 32/8/64 20.4 / 19.2, at 32/8/128 29.1 / 28.4, at
+ * 8/4/256 30.8 / 28.9; 333 over 800 keys at 32/8/128 29.7 / 33.8; 200 over 12K
+ * at 4/4/64 25.7 / 24.9. */
 static void plan(const LayerView &L, const tl_attn_args *a, u32 G, u32 cus, u32 &W, u32 &ns) {
     const u32 D = L.head_dim, bn = D <= 128 ? 64 : 32, GN = tasks_per_block(D, G);
-    const float part_us = (float)a->n * a->n_head * D * 4.f * 2.f / 5e6f;   /* per split */
+    const float part_us = 0.11f + (float)a->n * a->n_head * D * 4.f * 2.f / 6.1e6f;   /* per split */
     float best = 0.f;
     W = 0;
     for (u32 w = 8; w >= 4; w -= 4) {
-        const float tile = L.q8 ? 2.1f : D == 64 ? (w == 8 ? 1.18f : 0.94f)
-                                       : D == 128 ? (w == 8 ? 1.70f : 1.55f) : (w == 8 ? 1.39f : 1.5f);
+        const float tile = tile_us(D, w, L.q8), start = w == 8 && D <= 128 ? 3.f : 0.f;
         const u32 base = task_blocks(a->n, GN, w) * L.n_kv_head;
         if (base > cus && W) break;
         const u32 rows = ((w - 1) / GN + 1) * 32;
@@ -263,7 +281,7 @@ static void plan(const LayerView &L, const tl_attn_args *a, u32 G, u32 cus, u32 
         const u32 most = base < cus ? cus / base : 1u;
         for (u32 k = 1; k <= most; k++) {
             const u32 tiles = ((span + k - 1) / k + bn - 1) / bn;
-            const float t = tiles * tile + (w == 8 && D <= 128 ? 3.f : 0.f) + (k > 1 ? 5.f + k * part_us : 0.f);
+            const float t = tiles * tile + start + (k > 1 ? 3.5f + k * part_us : 0.f);
             if (!W || t < best) {
                 best = t;
                 W = w;
