@@ -128,3 +128,43 @@ def test_split_merge_paths_agree(T, case):
     want = run(kernel=1)
     for got in (run(), run(single=1), run(polls=1)):
         assert (got - want).abs().max().item() < 64 * 2.0 ** -24 * 5
+
+
+def test_unequal_sessions_share_cache_lines(T):
+    """Rows of 64 bytes (Q8_0 at head_dim 64) lie two to a cache line, their
+    scales 32 to one: through permuted slot tables a group's splits share
+    lines, so the plan for unequal lengths keeps a group on one L2, as the
+    plan with 240 workgroups (10 equal splits of 24 groups) does.  Measured
+    0.96 of the latter's time; 1.16 with the splits spread over the L2s."""
+    import tlkv
+    lib, g, keep = tlkv.lib(), T.Generator(device="cuda"), []
+    g.manual_seed(1)
+    n_head, n_kv, hd, lens = 32, 8, 64, [15000, 20000, 17321]
+
+    def batch():
+        seqs = []
+        for pos in lens:
+            L = tlkv.LayerQ8(pos + 1, n_kv, hd)
+            sl = T.randperm(pos + 1, generator=g, device="cuda").to(T.int32)
+            q, k, v = (T.randn((1, h * hd), generator=g, device="cuda") for h in (n_head, n_kv, n_kv))
+            out = T.zeros_like(q)
+            keep.append((L, sl, q, k, v, out))
+            seqs.append(tlkv.DecodeSeqQ8(L.desc, sl.data_ptr(), pos, 0, q.data_ptr(), k.data_ptr(),
+                                         v.data_ptr(), out.data_ptr()))
+        return (tlkv.DecodeSeqQ8 * len(lens))(*seqs)
+
+    arrs, times = [batch() for _ in range(8)], []
+    for wgs in (0, 240):
+        with tlkv.tuning(tlkv.TUNE_DECODE_WGS, wgs):
+            t = []
+            for _ in range(8):
+                e0, e1 = (T.cuda.Event(enable_timing=True) for _ in range(2))
+                e0.record()
+                for arr in arrs * 3:
+                    tlkv.check(lib.tl_attn_decode_batch_q8(arr, len(lens), n_head, 0, hd ** -0.5,
+                                                           tlkv.stream_handle()))
+                e1.record()
+                T.cuda.synchronize()
+                t.append(e0.elapsed_time(e1))
+        times.append(min(t))
+    assert times[0] < 1.08 * times[1], times

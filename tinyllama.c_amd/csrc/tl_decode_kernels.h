@@ -908,16 +908,20 @@ __device__ __attribute__((always_inline)) inline void decode_ring_body(const Dec
 
     u32 n_split = p.n_split;
     const u32 bid = blockIdx.x;
-    u32 grp, split, wg_grp;   /* group, split, the group's first workgroup (partials) */
+    u32 grp, split, wg_grp;   /* group, split, workgroups of the groups before it (partials) */
     if constexpr (RAGGED) {
         u32 s = 0;
 #pragma unroll
         for (u32 i = 1; i < TL_MAX_BATCH_SEQ; i++) s += bid >= p.wg0[i] ? 1u : 0u;
         const u32 w0 = p.wg0[s], local = bid - w0;
         n_split = (p.wg0[s + 1] - w0) / p.n_kv;
-        split = local % n_split;
-        grp = s * p.n_kv + local / n_split;
-        wg_grp = bid - split;
+        /* a session's workgroups go through its kv-heads first, so with 8 of
+         * them a group's splits are on one XCD (workgroup b runs on XCD b % 8),
+         * as below */
+        const u32 kv = local % p.n_kv;
+        split = local / p.n_kv;
+        grp = s * p.n_kv + kv;
+        wg_grp = w0 + kv * n_split;
     } else {
         const u32 n_groups = gridDim.x / n_split;
         if ((n_groups & 7) == 0) {
