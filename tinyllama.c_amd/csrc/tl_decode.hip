@@ -242,8 +242,17 @@ static int launch_decode(DecParams &p, u32 n_rows_total, u32 head_dim, u32 G, u3
             else lo = mid + 1;
         }
         const u32 most = (max_vis + hi - 1) / hi;
-        /* worth it from a sixth fewer keys on */
-        if (hi <= chunk - chunk / 6 && (!any_staged || hi <= TL_DEC_MAX_CHUNK) && most <= TL_MERGE_MAX_SPLIT_DIST && G * most <= 2048 &&
+        /* Worth it from a quarter fewer keys on, over a Q8_0 cache from a sixth
+         * (there a workgroup's share of the keys bounds the launch, over f16
+         * rows the bandwidth of all of them does more).  By length / equal, mean
+         * of 60 f16 and 65 Q8_0 batches of 2 to 12 sessions of 60 to 24K keys:
+         * f16, a sixth to a quarter fewer keys 1.005, a quarter to a third 0.985,
+         * a third to a half 0.93; Q8_0 0.96, 0.93, 0.87; less than a sixth 1.02,
+         * 0.99.  `target` holds for these instances too: one workgroup per CU,
+         * by its LDS (140 to 158 KB), as in the common kernel's. */
+        const u32 worth = q8 ? chunk - chunk / 6 : chunk - chunk / 4;
+        if (hi <= worth && (!any_staged || hi <= TL_DEC_MAX_CHUNK) &&
+            most <= TL_MERGE_MAX_SPLIT_DIST && G * most <= 2048 &&
             n_groups <= TL_MERGE_MAX_GROUPS && !tl_tune(TL_TUNE_DECODE_MERGE_KERNEL)) {
             p.ragged = 1;
             chunk = hi;
