@@ -560,6 +560,35 @@ def test_prefill_plan_counts_the_merge(T, case):
     assert times[0] < 1.2 * min(times[1:]), times
 
 
+def test_few_heads_and_very_many_keys_take_the_prefill_kernel(T):
+    """More keys than a folded decode group can merge the splits of: measured
+    5 times the prefill kernel's time on the decode kernel."""
+    import tlkv
+    n_head, n_kv, hd, pos, n = 1, 1, 64, 280000, 17
+    g = T.Generator(device="cuda")
+    g.manual_seed(n)
+    L = tlkv.Layer(pos + n, n_kv, hd)
+    sl = T.randperm(pos + n, generator=g, device="cuda").to(T.int32)
+    q, k, v = (T.randn((n, h * hd), generator=g, device="cuda") for h in (n_head, n_kv, n_kv))
+    times, outs = [], []
+    for kernel in (0, 2):
+        out = T.zeros_like(q)
+        a = tlkv.attn_args(q, k, v, out, sl, pos, n, n_head, hd, n_kv, 0, O.scale_of(hd))
+        with tlkv.tuning(tlkv.TUNE_NO_PREFILL, kernel):
+            t = []
+            for _ in range(6):
+                e0, e1 = (T.cuda.Event(enable_timing=True) for _ in range(2))
+                e0.record()
+                tlkv.check(tlkv.lib().tl_attn(L.desc, a, tlkv.stream_handle()))
+                e1.record()
+                T.cuda.synchronize()
+                t.append(e0.elapsed_time(e1))
+        times.append(min(t))
+        outs.append(out)
+    assert T.equal(outs[0], outs[1])
+    assert times[0] < 1.5 * times[1], times
+
+
 # windows that reach past the first key hide nothing, up to "no limit" as the
 # largest number and the last ones whose sum with a position passes 2^32
 @pytest.mark.parametrize("window", [2 ** 32 - 1, 2 ** 32 - 600, 2 ** 31, 900])

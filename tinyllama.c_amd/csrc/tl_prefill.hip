@@ -210,7 +210,16 @@ bool tl_prefill_supported(const LayerView &L, const tl_attn_args *a) {
  * 17.6 / 19.5, 2K 23.2 / 22.5, 4K 33.6 / 24.5; 32/8/64, 32 rows 4K 15.1 / 17.1,
  * 8K 20.3 / 20.5, 16K 29.4 / 23.7; 8/4/256, 32 rows 2K 21.5 / 22.7, 4K 29.9 /
  * 26.5.  Q8_0, 32 rows 1K 17.1 / 21.4, 2K 22.9 / 23.2, 4K 31.0 / 27.0; 8/4/256
- * 2K 24.8 / 24.8. */
+ * 2K 24.8 / 24.8.  One q-head per kv-head (where the line lies at more rows x
+ * keys), just below and just above it: 8/8/128, 17 rows 22K 29.2 / 28.0, 24K
+ * 31.0 / 29.2; 64 rows 5.8K 19.8 / 19.6, 6.4K 20.4 / 20.0; Q8_0, 32 rows 7.2K
+ * 22.4 / 23.5, 8K 23.4 / 23.8; 32/32/128, 64 rows 1.4K 19.8 / 18.8, 1.6K 20.9 /
+ * 18.5.  Few heads: 4/4/64, 32 rows 46K 24.2 / 26.3, 51K 25.2 / 27.3, 17 rows 55K
+ * 26.2 / 27.8, 87K 42.0 / 34.8; Q8_0, 64 rows 14K 21.1 / 23.3, 16K 21.6 / 23.7;
+ * 1/1/64, 64 rows 103K 19.3 / 32.5, 17 rows 221K 26.8 / 41.1 — but 349K 246 /
+ * 50: past TL_DEC_FOLD_MAX_KEYS the chunks of a slot table make more splits than
+ * a folded group merges (16 columns x 128), and each row reads the keys again. */
+#define TL_DEC_FOLD_MAX_KEYS (TL_DEC_MAX_CHUNK * 2048u / 16u)
 static u64 prefill_min_work(const LayerView &L) {
     const bool wide = L.head_dim == 256;
     if (L.q8) return wide ? 180000000u : 250000000u;
@@ -222,7 +231,7 @@ bool tl_use_prefill(const LayerView &L, const tl_attn_args *a) {
     if (tl_tune(TL_TUNE_NO_PREFILL) == 2) return true;
     const u64 keys = (u64)a->pos + a->n;
     const u64 vis = (a->window && keys > a->window) ? a->window : keys;
-    return a->n > TL_DEC_FOLD_MAX_ROWS ||
+    return a->n > TL_DEC_FOLD_MAX_ROWS || vis > TL_DEC_FOLD_MAX_KEYS ||
            (u64)a->n * vis * a->n_head * L.head_dim > prefill_min_work(L);
 }
 
