@@ -245,7 +245,7 @@ static u32 tasks_per_block(u32 D, u32 G) { return D == 256 ? G * pf_parts<256>()
  * workgroup's threads dequantize the tile, so half of them take longer), then
  * moved to where the plan's choices cost least over 260 shapes (65 to 1024 rows,
  * 0 to 14K keys, 1 to 32 heads, both caches), each timed at both widths and up
- * to 16 split counts: the choices are 1.5% from the best ones on average (4.1%
+ * to 16 split counts: the choices are 1.4% from the best ones on average (4.1%
  * with one Q8_0 cost for all and a merge that costs the same for any count), 7%
  * for one shape in 20.  At 256 (slopes 1.39 / 1.5, Q8_0 1.63 / 1.9) and for 4
  * waves over a Q8_0 cache short runs count for more than the slope. */
@@ -253,7 +253,7 @@ static float tile_us(u32 D, u32 w, bool q8) {
     if (q8) return D == 64 ? (w == 8 ? 1.12f : 1.45f) : D == 128 ? (w == 8 ? 1.90f : 2.10f)
                                                                  : (w == 8 ? 2.06f : 1.90f);
     return D == 64 ? (w == 8 ? 1.10f : 0.94f) : D == 128 ? (w == 8 ? 1.70f : 1.55f)
-                                                         : (w == 8 ? 1.39f : 1.19f);
+                                                         : (w == 8 ? 1.39f : 1.33f);
 }
 
 /* Waves per workgroup (W) and key splits of a launch, by a cost in us: the
@@ -279,11 +279,17 @@ static void plan(const LayerView &L, const tl_attn_args *a, u32 G, u32 cus, u32 
     const u32 D = L.head_dim, bn = D <= 128 ? 64 : 32, GN = tasks_per_block(D, G);
     const float part_us = 0.11f + (float)a->n * a->n_head * D * 4.f * 2.f / 6.1e6f;   /* per split */
     float best = 0.f;
+    u32 wide = 0;                              /* workgroups with 8 waves */
     W = 0;
     for (u32 w = 8; w >= 4; w -= 4) {
         const float tile = tile_us(D, w, L.q8), start = w == 8 && D <= 128 ? 3.f : 0.f;
         const u32 base = task_blocks(a->n, GN, w) * L.n_kv_head;
         if (base > cus && W) break;
+        /* no more workgroups with 4 waves: the other 4 at least stage the tiles
+         * (at head_dim 256: 17 rows over 8K keys at 8/4/256, 8 / 4 waves 26.4 /
+         * 27.5, Q8_0 28.2 / 30.3) */
+        if (W && D > 128 && base == wide) break;
+        wide = base;
         const u32 rows = ((w - 1) / GN + 1) * 32;
         u32 span = a->pos + a->n;              /* most keys any workgroup sees */
         if (a->window && span > (u64)a->window + rows) span = a->window + rows;
