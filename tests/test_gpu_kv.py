@@ -918,13 +918,17 @@ def test_two_host_threads_decode(T):
             assert np.abs(host(S["out"][t]) - ref).max() < TOL, f"session {i} step {t}"
 
 
-@pytest.mark.parametrize("shape", [(32, 8, 128, 8192, 8000), (28, 4, 128, 8300, 8192)])
+@pytest.mark.parametrize("shape", [(32, 8, 128, 8192, 8000), (28, 4, 128, 8300, 8192),
+                                   (16, 4, 128, 8300, 8192), (8, 1, 256, 1300, 1279)])
 def test_decode_split_merge_fallback(T, shape):
     """The split merge's bounded waits, forced from the host: with no polls
     every split gives up its slice and the last split of each group to
     arrive merges all of them; with one poll some do and some do not.  The
     outputs equal the default run's bit for bit (every slice is merged by
-    the same code from the same partials, whoever runs it)."""
+    the same code from the same partials, whoever runs it).  32 splits of 4
+    heads (the first shape) have too few bytes for slices: their last split
+    merges and nothing waits; the others have 64 splits of 7 and of 4 heads and
+    40 of 8 heads at head_dim 256."""
     import tlkv
     n_head, n_kv, hd, cap, pos = shape
     outs = []
@@ -937,12 +941,15 @@ def test_decode_split_merge_fallback(T, shape):
         assert np.array_equal(outs[0].view(np.uint32), o.view(np.uint32))
 
 
-@pytest.mark.parametrize("shape", [(32, 8, 128, 8200, 8000, 1), (32, 8, 128, 4200, 4000, 4)])
+@pytest.mark.parametrize("shape", [(32, 8, 128, 8200, 8000, 1), (32, 8, 128, 4200, 4000, 4),
+                                   (28, 4, 128, 8300, 8192, 1)])
 def test_decode_graph_replay(T, shape):
     """OP_ATTN captured in a HIP graph and replayed: each replay, with new q
     written eagerly between replays, equals the eager call on the same
     inputs bit for bit and the oracle within tolerance (the split merge's
-    state carries nothing from one replay into the next)."""
+    state carries nothing from one replay into the next).  The first shape's
+    groups are merged by their last split, the others' in slices by every
+    split (32 splits of 16 columns, 64 of 7)."""
     import tlkv
     n_head, n_kv, hd, cap, pos, n = shape
     rng = np.random.default_rng(pos + n)
