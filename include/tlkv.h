@@ -125,7 +125,9 @@ int tl_init(int device);
 #define TL_TUNE_DECODE_SINGLE_MERGE 5   /* 1: the last split of a group merges all of it */
 #define TL_TUNE_DECODE_MERGE_POLLS  6   /* n: at most n - 1 polls per wait of the split merge */
 #define TL_TUNE_PREFILL_APPEND_POLLS 7  /* n: at most n - 1 polls per wait for the fused append */
-#define TL_TUNE_PREFILL_SEPARATE_APPEND 8 /* 1: prefill batches append in a launch of their own */
+#define TL_TUNE_PREFILL_SEPARATE_APPEND 8 /* 1: prefill batches append in a launch of their own
+                                           (with RoPE the rotating launch does in any case,
+                                           and keys 7 and 8 change nothing) */
 #define TL_TUNE_DECODE_MFMA         9   /* 1: decode tiles on the vector ALUs, 2: on the matrix cores */
 #define TL_TUNE_DECODE_ROWS        10   /* n: batch rows per matrix-core decode group (1: one) */
 #define TL_TUNE_COUNT               11

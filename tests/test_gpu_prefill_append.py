@@ -1,15 +1,17 @@
 """OP_ATTN on prefill batches with the append fused into the prefill launch:
-the launch's workgroups write the batch rows (f32 -> f16 RNE, K rotated when
-RoPE is fused) into the cache before any of them reads it, each publishing
-its 16-row units with a flag; a workgroup whose keys reach the batch rows
-waits (bounded) for the flags and reads those rows back device-coherently,
-and writes a unit itself when its flag does not come.
+the launch's workgroups write the batch rows (f32 -> f16 RNE) into the cache
+before any of them reads it, each publishing its 16-row units with a flag; a
+workgroup whose keys reach the batch rows waits (bounded) for the flags and
+reads those rows back device-coherently, and writes a unit itself when its
+flag does not come.  With RoPE a launch before the attention launch rotates
+and writes them, and nothing waits.
 
 Checked against the separate append launch (the previous path) on twin
 layers: the cache contents and the outputs are the same bits, with the
 bounded wait as usual and with no wait at all (every workgroup writes every
 unit it reads itself: the fallback), and the outputs are within 2e-3 of the
-oracle (src/backend/cpu/cpu_op.c:995-1062).  Shapes: config 4's chunk at
+oracle (src/backend/cpu/cpu_op.c:995-1062).  With RoPE the separate path
+rotates q and K and appends in launches of their own.  Shapes: config 4's chunk at
 depth with a permuted slot table and several key splits, config 4's first
 chunk (every key is a batch row), gqa 7, head_dim 64 and 256, a window on a
 ring, a ragged batch, and the fused-RoPE entry point."""
@@ -51,7 +53,8 @@ CASES = [
 
 
 def _run(T, case, mode):
-    """mode: 'separate' (own append launch), 'fused', 'fallback' (no wait)."""
+    """mode: 'separate' (own append launch, after tl_rope with RoPE), 'fused',
+    'fallback' (no wait; not with RoPE, where nothing waits)."""
     import tlkv
     nh, nkv, hd, cap, pos, n, win, ring, perm, rope = case
     rng = np.random.default_rng(pos + n + hd)
@@ -77,6 +80,13 @@ def _run(T, case, mode):
     with sep, polls:
         if rope is None:
             tlkv.check(lib.tl_attn(L.desc, a, None))
+        elif mode == "separate":
+            qr, kr = dev(T, q), dev(T, k)
+            for x, w, heads in ((qr, qd, nh), (kr, kd, nkv)):
+                tlkv.check(lib.tl_rope(tlkv.ptr(x), n, w, heads, hd, hd, pos, rope[1], rope[0], None))
+            ar = tlkv.attn_args(qr, kr, dev(T, v), out, ds, pos, n, nh, hd, nkv, win, O.scale_of(hd))
+            tlkv.check(lib.tl_kv_append(L.desc, tlkv.ptr(kr), ar.v, kd, tlkv.ptr(ds), pos, n, None))
+            tlkv.check(lib.tl_attn_noappend(L.desc, ar, None))
         else:
             rp = tlkv.RopeParams(hd, rope[1], rope[0])
             tlkv.check(lib.tl_attn_rope(L.desc, a, rp, None))
@@ -114,7 +124,7 @@ LONG_CASES = [
 def test_fused_append_equals_separate(T, case):
     base = _run(T, case, "separate")
     assert np.abs(base["out"] - base["ref"]).max() < TOL
-    for mode in ("fused", "fallback"):
+    for mode in ("fused", "fallback") if case[-1] is None else ("fused",):
         got = _run(T, case, mode)
         assert np.array_equal(got["k"], base["k"]), f"{mode}: K cache differs"
         assert np.array_equal(got["v"], base["v"]), f"{mode}: V cache differs"
