@@ -56,7 +56,7 @@ def test_attn_rope_equals_rope_then_attn(T, case):
 
 # prefill batches at the edges of the rotating pre-launch: partial rotation,
 # a half-head that is no multiple of 8 elements (NEOX), heads that do and do
-# not fill its workgroups' passes
+# not fill its workgroups' passes, more rows than its grid (2048 workgroups)
 PREP_CASES = [
     (8, 8, 128, 3, 290, 128, 1, 5e5),
     (8, 8, 64, 77, 257, 64, 0, 5e5),
@@ -66,6 +66,9 @@ PREP_CASES = [
     (8, 2, 256, 1, 31, 24, 1, 1e4),
     (8, 1, 64, 500, 17, 2, 1, 1e4),
     (64, 8, 256, 20, 18, 256, 1, 1e4),
+    (4, 2, 64, 5, 2100, 64, 1, 1e4),
+    (6, 1, 128, 0, 4097, 36, 1, 1e6),
+    (8, 4, 256, 7, 2050, 64, 0, 5e5),
 ]
 
 

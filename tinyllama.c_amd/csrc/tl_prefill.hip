@@ -56,8 +56,8 @@ TL_PREFILL_PICKER(tl_prefill_fn, false)
  * heads, while the row's loads are in flight.  The f16 q goes where the
  * attention output will be (the first half of each head's D floats of dst),
  * so nothing is allocated; the attention launch reads it before that output
- * is written.  The lanes of one head are of one wave and load before they
- * store, so dst may be q.
+ * is written.  dst may be q: the D/8 lanes of one head are of one wave, and
+ * every read of the head is before its stores (the wave barrier).
  *
  * Bound by latency: one round trip for the row beside one sincosf, then the
  * stores.  Rotated inside the attention launch instead, every key split and
@@ -123,6 +123,11 @@ __global__ __launch_bounds__(256) void attn_rope_prep_kernel(const PrepParams p)
                     else
                         rope8_tab_any(x[u], src_of(i), e0, p.rope.rdim, s_tab);
                 }
+                /* in place (dst = q) the stores below replace elements that other
+                 * lanes of the head rotate with (read above, or just now for a
+                 * half that is no multiple of 8): no lane stores before all of
+                 * them have read, also where lanes past rope_dim read nothing */
+                __builtin_amdgcn_wave_barrier();
                 if (hd < p.n_head) {
                     const float sc = p.scale_log2;
                     u16 *o = (u16 *)(p.dst + (u64)row * p.q_stride + (u64)hd * D) + e0;

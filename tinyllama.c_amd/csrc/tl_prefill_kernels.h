@@ -62,6 +62,7 @@ __global__ __attribute__((amdgpu_flat_work_group_size(64 * W, 64 * W), amdgpu_wa
     constexpr int CPR = D / 8;           /* 16-byte chunks per row */
     constexpr int KS = D / 16;           /* k-steps of the QK MFMA */
     constexpr int NP = pf_parts<D>();
+    static_assert(W % NP == 0, "the waves of a row block and head share a workgroup");
     constexpr int DB = D / 32 / NP;      /* 32-row d-blocks of O^T of a wave */
     constexpr int KB = BN / 32;          /* 32-key blocks of S^T per tile */
     constexpr int UNITS = BN * CPR;      /* 16-byte units per K (or V) tile */
@@ -160,8 +161,12 @@ __global__ __attribute__((amdgpu_flat_work_group_size(64 * W, 64 * W), amdgpu_wa
 
     /* Q operand: lane holds Q[row lr][16s + 8h .. +8], f16, log2-scaled: from
      * the f32 rows, or as attn_rope_prep_kernel left it in dst (f16 at the
-     * start of each row's head; this wave alone reads these rows and heads,
-     * before it or the merge writes them) */
+     * start of each row's head, where part 0 of the head's output goes).  The
+     * NP waves that read a row block and head are neighbours in one workgroup
+     * (W, t0 and GN are multiples of NP) and have it in registers (the pin
+     * below) before the tile loop's first barrier; they write dst after the
+     * loop, or the merge launch does.  With key splits other workgroups read
+     * the same q and none writes dst */
     half8_t qop[KS];
     if (p.q) {
         const float *qrow = p.q + (u64)(row_ok ? my_q : 0) * p.q_stride + (u64)hq * D;
