@@ -218,10 +218,11 @@ static int launch_decode(DecParams &p, u32 n_rows_total, u32 head_dim, u32 G, u3
      * chunk whose workgroups still fit the rounds that the equal split takes
      * (its workgroups of the short sessions would have no keys, while the long
      * sessions' had max_vis / n_split).  8 sessions of 512 to 8192 keys at
-     * 28/4/128: 21.4 us per launch with equal counts, 17.7 by length. */
-    p.ragged = 0;
+     * 28/4/128: 21.4 us per launch with equal counts, 17.7 by length.  Not with
+     * RoPE over a Q8_0 cache: no entry point decodes several such sessions. */
+    bool ragged = false;
     u64 grid = (u64)n_split * n_groups;
-    if (rows == 1 && n_rows_total > 1 && n_split > 1 &&
+    if (rows == 1 && n_rows_total > 1 && n_split > 1 && !(q8 && p.rope.rdim) &&
         mf == tl_decode_matrix_tile((int)head_dim, (int)G, q8)) {
         const u32 n_seq = n_rows_total;
         u32 vis[TL_MAX_BATCH_SEQ];
@@ -254,7 +255,7 @@ static int launch_decode(DecParams &p, u32 n_rows_total, u32 head_dim, u32 G, u3
         if (hi <= worth && (!any_staged || hi <= TL_DEC_MAX_CHUNK) &&
             most <= TL_MERGE_MAX_SPLIT_DIST && G * most <= 2048 &&
             n_groups <= TL_MERGE_MAX_GROUPS && !tl_tune(TL_TUNE_DECODE_MERGE_KERNEL)) {
-            p.ragged = 1;
+            ragged = true;
             chunk = hi;
             n_split = most;
             u32 w = 0;
@@ -263,7 +264,7 @@ static int launch_decode(DecParams &p, u32 n_rows_total, u32 head_dim, u32 G, u3
                 if (i < n_seq) w += (vis[i] + chunk - 1) / chunk * p.n_kv;
             }
             grid = w;
-            K = q8 ? tl_pick_decode_rag_q8((int)head_dim, (int)G, p.rope.rdim != 0)
+            K = q8 ? tl_pick_decode_rag_q8((int)head_dim, (int)G)
                    : tl_pick_decode_rag((int)head_dim, (int)G, p.rope.rdim != 0);
         }
     }
@@ -300,7 +301,7 @@ static int launch_decode(DecParams &p, u32 n_rows_total, u32 head_dim, u32 G, u3
                          grid <= resident && !tl_tune(TL_TUNE_DECODE_SINGLE_MERGE)
                      ? dist_min : 0u;
         p.dist_groups = (u32)n_groups;
-        if (p.ragged) {
+        if (ragged) {
             p.dist_groups = 0;
             for (u32 i = 0; i < n_rows_total; i++)
                 if (p.wg0[i + 1] - p.wg0[i] >= dist_min * p.n_kv) p.dist_groups += p.n_kv;

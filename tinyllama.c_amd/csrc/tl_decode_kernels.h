@@ -1762,7 +1762,7 @@ __global__ __launch_bounds__(64 * TL_RING_WAVES) void attn_decode_ring_kernel_s1
     decode_ring_body<D, G, ROPE, false, MF, true, false>(p);
 }
 
-/* Batches of sessions of unequal lengths (DecParams.ragged): an instance of
+/* Batches of sessions of unequal lengths (DecParams.wg0): an instance of
  * its own, because the lookup of a workgroup's session and split cost every
  * other launch 0.3 us (decode at 32/8/64 over 700 keys 8.1 -> 8.4). */
 template <int D, int G, bool ROPE, bool Q8, bool MF>
@@ -1797,6 +1797,6 @@ DecKernel tl_pick_decode_q8(int D, int G, bool rope, bool mf);
 /* the u16-slot instances (f16 cache, matrix-core tile; tl_decode_s16.hip) */
 DecKernel tl_pick_decode_s16(int D, int G, bool rope);
 /* the unequal-length instances, tile as tl_decode_matrix_tile (tl_decode_rag.hip,
- * tl_decode_rag_q8.hip) */
+ * tl_decode_rag_q8.hip: without RoPE only) */
 DecKernel tl_pick_decode_rag(int D, int G, bool rope);
-DecKernel tl_pick_decode_rag_q8(int D, int G, bool rope);
+DecKernel tl_pick_decode_rag_q8(int D, int G);

@@ -66,10 +66,10 @@ struct DecParams {
     uint32_t dist;           /* n > 0: in groups of at least n splits every split merges its
                                 own slice of the output */
     uint32_t polls;          /* most polls per bounded wait of the split merge */
-    /* sessions of unequal lengths: each has as many splits of `chunk` keys as
-     * it fills; session i's workgroups are [wg0[i], wg0[i + 1]), n_kv groups of
-     * equal split counts (n_split is the largest).  0: every group n_split */
-    uint32_t ragged;
+    /* sessions of unequal lengths (attn_decode_ring_kernel_rag): each has as
+     * many splits of `chunk` keys as it fills; session i's workgroups are
+     * [wg0[i], wg0[i + 1]), n_kv groups of equal split counts (n_split is the
+     * largest) */
     uint32_t wg0[TL_MAX_BATCH_SEQ + 1];
     uint32_t dist_groups;    /* groups whose splits merge slices (dist) */
     uint32_t rows_per_wg;    /* matrix-core tile: batch rows per workgroup group (their
