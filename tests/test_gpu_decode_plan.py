@@ -110,8 +110,9 @@ MERGES = [(32, 8, 128, 64 * n, 64) for n in (2, 8, 9, 16, 17, 23, 24, 32)] + [
     (8, 2, 64, 128 * 64, 128)]
 
 
-@pytest.mark.parametrize("case", MERGES)
-def test_split_merge_paths_agree(T, case):
+def _merge_runs(T, case, wgs=0):
+    """The partials of one launch merged by the separate launch, then as the
+    plan has it, by each group's last workgroup, and with no waits."""
     import tlkv
     n_head, n_kv, hd, keys, per = case
     lib = tlkv.lib()
@@ -123,7 +124,7 @@ def test_split_merge_paths_agree(T, case):
     def run(**tune):
         out = T.full_like(q, float("nan"))
         a = tlkv.attn_args(q, None, None, out, None, keys - 1, 1, n_head, hd, n_kv, 0)
-        with tlkv.tuning(tlkv.TUNE_DECODE_MIN_KEYS, per), \
+        with tlkv.tuning(tlkv.TUNE_DECODE_MIN_KEYS, per), tlkv.tuning(tlkv.TUNE_DECODE_WGS, wgs), \
              tlkv.tuning(tlkv.TUNE_DECODE_MERGE_KERNEL, tune.get("kernel", 0)), \
              tlkv.tuning(tlkv.TUNE_DECODE_SINGLE_MERGE, tune.get("single", 0)), \
              tlkv.tuning(tlkv.TUNE_DECODE_MERGE_POLLS, tune.get("polls", 0)):
@@ -132,9 +133,37 @@ def test_split_merge_paths_agree(T, case):
         T.cuda.synchronize()
         return out
 
-    want = run(kernel=1)
-    for got in (run(), run(single=1), run(polls=1)):
+    return run(kernel=1), (run(), run(single=1), run(polls=1))
+
+
+@pytest.mark.parametrize("case", MERGES)
+def test_split_merge_paths_agree(T, case):
+    want, gots = _merge_runs(T, case)
+    for got in gots:
         assert (got - want).abs().max().item() < 64 * 2.0 ** -24 * 5
+
+
+# more splits than a wave has lanes, where the last workgroup's merge depends on
+# the columns: shared by 16, 2 and 1 threads per column, shares from LDS (from 97
+# splits on at head_dim 64), more than the 256 splits whose pairs are read at
+# once; and two trips of few columns, where slices begin (33 splits of 7 heads,
+# 49 of 5 at head_dim 64)
+MANY = [(1, 1, 64, 128 * n, 128) for n in (65, 75, 224)] + [
+    (7, 1, 64, 128 * n, 128) for n in (32, 33, 65, 96, 97)] + [
+    (5, 1, 64, 128 * 48, 128), (5, 1, 64, 128 * 49, 128), (4, 2, 64, 128 * 128, 128),
+    (1, 1, 128, 64 * 256, 64), (2, 1, 256, 32 * 200, 32), (4, 1, 256, 32 * 100, 32),
+    (8, 1, 256, 32 * 100, 32), (7, 1, 128, 64 * 235, 64),
+    (4, 1, 128, 64 * 256, 64), (4, 1, 128, 64 * 257, 64), (4, 1, 128, 64 * 500, 64),
+    (1, 1, 64, 128 * 400, 128), (4, 1, 64, 128 * 300, 128)]
+
+
+@pytest.mark.parametrize("case", MANY)
+def test_many_splits_merged_alike(T, case):
+    """As above, the f32 sums over up to 500 splits."""
+    n_split = case[3] // case[4]
+    want, gots = _merge_runs(T, case, 1024)
+    for got in gots:
+        assert (got - want).abs().max().item() < max(64, n_split) * 2.0 ** -24 * 5
 
 
 def test_unequal_sessions_share_cache_lines(T):

@@ -178,7 +178,7 @@ static int launch_decode(DecParams &p, u32 n_rows_total, u32 head_dim, u32 G, u3
      * 128 9.2; of 4 kv-heads over 500 keys 8.6 / 9.5 (Q8_0 9.5 / 10.6), over
      * 1100 10.7 / 10.1, 94 keys 8.4 / 6.9; 256, a 1024-key window: 32 keys 9.4,
      * 128 10.4 */
-    const u32 one_trip = 8;
+    const u32 one_trip = TL_MERGE_TRIP;
     const u32 half_waves = waves / 2 * tk;
     u32 min_keys = tuned(TL_TUNE_DECODE_MIN_KEYS, half_waves);
     if (head_dim == 128 && !tl_tune(TL_TUNE_DECODE_MIN_KEYS)) {
@@ -295,7 +295,9 @@ static int launch_decode(DecParams &p, u32 n_rows_total, u32 head_dim, u32 G, u3
         const u64 resident = (u64)resident_per_cu(K.fn, K.threads) * cu_count();
         const u32 cols4 = R * G * head_dim / 4;      /* output float4s of a group */
         u32 dist_min = TL_MERGE_MIN_SPLIT_DIST;
-        dist_min = umax(dist_min, (TL_MERGE_MIN_BYTES_DIST + cols4 * 16 - 1) / (cols4 * 16));
+        dist_min = umax(dist_min, cols4 <= (u32)K.threads / 4
+                                      ? TL_MERGE_TRIP * ((u32)K.threads / cols4) + 1
+                                      : (TL_MERGE_MIN_BYTES_DIST + cols4 * 16 - 1) / (cols4 * 16));
         dist_min = umax(dist_min, (cols4 + TL_MERGE_SLICE_MAX - 1) / TL_MERGE_SLICE_MAX);
         p.dist = in_kernel_merge && n_split >= dist_min && n_split <= TL_MERGE_MAX_SPLIT_DIST &&
                          grid <= resident && !tl_tune(TL_TUNE_DECODE_SINGLE_MERGE)

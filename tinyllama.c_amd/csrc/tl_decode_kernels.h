@@ -670,28 +670,112 @@ constexpr int pow2_floor(int x) { return x >= 16 ? 16 : x >= 8 ? 8 : x >= 4 ? 4 
 
 /* Merge of a group's ns partials by its last workgroup:
  * out = sum_s exp2(m_s - M) acc_s / sum_s exp2(m_s - M) l_s per output float4
- * (head h, dims d..d+3; ncol heads, ncol * D/4 <= NT float4s).  Bound by the
- * round trips of its device-coherent loads.  Few float4s and many splits: the
- * threads cover the float4s P times over (P shares of the splits, consecutive
- * lanes on consecutive 16 bytes of one split's row), so all rows are requested
- * in one trip, one wave per head turns the (m, l) pairs into weights meanwhile,
- * and the shares add through LDS.  Otherwise each thread folds all splits with
- * an online max, K rows per trip.  us per launch, shares / fold: 32 splits of
- * 4 heads at head_dim 128 over 32K keys 28.1 / 28.5, over 4K 10.2 / 10.6; of 2
- * heads at 256 9.4 / 9.6; but 32 splits of 7 heads at 128 (P = 2) 10.6 / 10.1,
- * and 16 splits of 4 heads at 64 9.2 / 8.7 (two trips fold them).
- * s_buf: ncol * ns <= 2048 pairs, then the shares. */
-template <int D, int NT>
-TL_DEV void split_merge_regs(const DecParams &p, u32 pb, const float2 *ml_g, u32 ns, u32 kvh,
+ * (column: head h, dims d..d+3; ncol heads).  Bound by the round trips of its
+ * device-coherent loads and, past 64 splits, by what one CU can request.  Two
+ * ways, each faster on its side:
+ * split_merge_fold: TPC neighbouring threads per column fold their shares of
+ * the splits with an online max, 8 rows per trip, and combine by DPP.
+ * split_merge_shares, from 17 splits of at most NT / 4 columns on: the threads
+ * cover the columns P times over (consecutive lanes on consecutive 16 bytes of
+ * one split's row), one wave per head turns the (m, l) pairs into weights while
+ * the rows are on their way, and the shares add through LDS.
+ * us per launch, shares / fold by one thread: 32 splits of 4 heads at head_dim
+ * 128 over 32K keys 28.1 / 28.5, over 4K 10.2 / 10.6; of 2 heads at 256 9.4 /
+ * 9.6; but 32 splits of 7 heads at 128 (P = 2) 10.6 / 10.1, and 16 splits of 4
+ * heads at 64 9.2 / 8.7 (two trips fold them).  At 64 two threads per column
+ * fold 9 to 16 splits in one trip (16 of 4 heads 7.1, by one thread 7.4);
+ * elsewhere one is as fast or faster (16 of 2 heads at 256 8.3, by four 8.6).
+ * Past 64 splits, shares / fold by TPC threads: 75 splits of one head at 64 (TPC
+ * 16) 8.4 / 7.1, of 7 (TPC 2) 10.4 / 9.7, of 4 9.3 / 8.9; 110 of 7 11.4 / 11.0, of
+ * 4 9.6 / 10.2; 224 of 4 12.8 / 15.3; 200 of 4 at 128 (TPC 1) 15.5 / 19.6; 200 of 2
+ * at 256 (TPC 4) 16.4 / 20.0; with more columns (P = 2) 235 of 4 at 256 (TPC 2)
+ * 27.6 / 23.6.
+ * s_buf: ncol * ns <= 2048 pairs, then (shares) 1/L per head and the shares. */
+template <int D, int NT, int TPC>
+TL_DEV void split_merge_fold(const DecParams &p, u32 pb, const float2 *ml_g, u32 ns, u32 kvh,
                              u32 r, u32 gh, u32 ncol, const DecSeq &sq, float2 *s_buf) {
     constexpr float NEG_INF = -__builtin_huge_valf();
-    constexpr u32 K = 8;                       /* splits per load batch */
+    constexpr u32 K = TL_MERGE_TRIP;           /* splits per load batch */
+    const u32 tid = threadIdx.x, part = tid % TPC, col = tid / TPC;
+    const u32 h = col / (D / 4), d = (col % (D / 4)) * 4;
+    const bool mine = h < ncol;
+    const __amdgpu_buffer_rsrc_t rml = buf_rsrc(ml_g);
+    const __amdgpu_buffer_rsrc_t racc = buf_rsrc(p.ws_acc + (u64)pb * D);
+    u32x4v_t a[K];
+    auto load_batch = [&](u32 s0) __attribute__((always_inline)) {
+#pragma unroll
+        for (u32 k = 0; k < K; k++) {
+            const u32 s = min(s0 + k * TPC, ns - 1);
+            a[k] = __builtin_amdgcn_raw_buffer_load_b128(racc, ((h * ns + s) * D + d) * 4, 0, TL_SC1);
+        }
+    };
+    if (mine) load_batch(part);
+    for (u32 i = tid; i < ncol * ns; i += NT) {
+        const u32x2v_t ml = __builtin_amdgcn_raw_buffer_load_b64(rml, i * 8, 0, TL_SC1);
+        s_buf[i] = make_float2(__uint_as_float(ml[0]), __uint_as_float(ml[1]));
+    }
+    __asm__ volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    __syncthreads();
+    if (!mine) return;                         /* whole groups of TPC lanes */
+    float4 O = make_float4(0.f, 0.f, 0.f, 0.f);
+    float M = NEG_INF, L = 0.f;
+    const float2 *mlh = s_buf + h * ns;
+    for (u32 s0 = part; s0 < ns; s0 += K * TPC) {
+        if (s0 != part) load_batch(s0);
+        float2 ml[K];
+        float bm = NEG_INF;
+#pragma unroll
+        for (u32 k = 0; k < K; k++) {
+            const u32 s = s0 + k * TPC;
+            ml[k] = mlh[min(s, ns - 1)];
+            if (s >= ns) ml[k] = make_float2(NEG_INF, 0.f);   /* past the last split */
+            bm = fmaxf(bm, ml[k].x);
+        }
+        const float nm = fmaxf(M, bm);
+        const float mu = (nm == NEG_INF) ? 0.f : nm;
+        const float sc = fast_exp2(M - mu);
+        L *= sc;
+        O.x *= sc; O.y *= sc; O.z *= sc; O.w *= sc;
+        M = nm;
+#pragma unroll
+        for (u32 k = 0; k < K; k++) {
+            const float w = fast_exp2(ml[k].x - mu);
+            L = fmaf(w, ml[k].y, L);
+            O.x = fmaf(w, __uint_as_float(a[k][0]), O.x);
+            O.y = fmaf(w, __uint_as_float(a[k][1]), O.y);
+            O.z = fmaf(w, __uint_as_float(a[k][2]), O.z);
+            O.w = fmaf(w, __uint_as_float(a[k][3]), O.w);
+        }
+    }
+    if constexpr (TPC > 1) {
+        const float Mg = group_max<TPC>(M);
+        const float e = fast_exp2(M - ((Mg == NEG_INF) ? 0.f : Mg));
+        L = group_sum<TPC>(L * e);
+        O.x = group_sum<TPC>(O.x * e);
+        O.y = group_sum<TPC>(O.y * e);
+        O.z = group_sum<TPC>(O.z * e);
+        O.w = group_sum<TPC>(O.w * e);
+    }
+    if (part == 0) {
+        const float inv = 1.0f / L;
+        *(float4 *)&sq.dst[(u64)(r + h / gh) * p.q_stride + (u64)(kvh * gh + h % gh) * D + d] =
+            make_float4(O.x * inv, O.y * inv, O.z * inv, O.w * inv);
+    }
+}
+
+template <int D, int NT, bool MANY>
+TL_DEV void split_merge_shares(const DecParams &p, u32 pb, const float2 *ml_g, u32 ns, u32 kvh,
+                               u32 r, u32 gh, u32 ncol, const DecSeq &sq, float2 *s_buf) {
+    constexpr float NEG_INF = -__builtin_huge_valf();
+    constexpr u32 K = TL_MERGE_TRIP;           /* splits per load batch */
     const u32 tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    const u32 COLS = ncol * (D / 4);
-    const u32 P = ns > 2 * K && COLS <= NT / 4 ? (u32)NT / COLS : 1u;
+    const u32 COLS = ncol * (D / 4);           /* <= NT / 4, so ncol <= NT / 64 */
+    static_assert(NT / D <= NT / 64, "a wave per head");
+    const u32 P = (u32)NT / COLS;
     const u32 part = (tid / (D / 4)) / ncol, h = (tid / (D / 4)) % ncol, d = (tid % (D / 4)) * 4;
     const __amdgpu_buffer_rsrc_t rml = buf_rsrc(ml_g);
     const __amdgpu_buffer_rsrc_t racc = buf_rsrc(p.ws_acc + (u64)pb * D);
+    float *const s_w = (float *)s_buf;
     float *const s_inv = (float *)(s_buf + 2048);
     float4 *const s_o = (float4 *)(s_inv + 64);
     u32x4v_t a[K];
@@ -703,102 +787,88 @@ TL_DEV void split_merge_regs(const DecParams &p, u32 pb, const float2 *ml_g, u32
         }
     };
     float4 O = make_float4(0.f, 0.f, 0.f, 0.f);
-    float inv = 0.f;
-    if (P > 1) {
-        auto pair = [&](u32 hh, u32 s) {
-            const u32x2v_t v = __builtin_amdgcn_raw_buffer_load_b64(rml, (hh * ns + min(s, ns - 1)) * 8, 0, TL_SC1);
-            return make_float2(s < ns ? __uint_as_float(v[0]) : NEG_INF, __uint_as_float(v[1]));
+    /* lane i of wave h: splits i, i + 64, ... of head h; MANY (past 64 splits):
+     * four at once, in turn each costs a round trip */
+    constexpr u32 KP = MANY ? 4 : 1;
+    float2 ml[KP];
+    auto pair = [&](u32 s) __attribute__((always_inline)) {
+        const u32x2v_t v = __builtin_amdgcn_raw_buffer_load_b64(rml, (wave * ns + min(s, ns - 1)) * 8, 0, TL_SC1);
+        return make_float2(s < ns ? __uint_as_float(v[0]) : NEG_INF, __uint_as_float(v[1]));
+    };
+    if (wave < ncol) {
+#pragma unroll
+        for (u32 j = 0; j < KP; j++) ml[j] = pair(lane + 64 * j);
+    }
+    if (part < P) load_batch(part);
+    if (wave < ncol) {
+        float M = NEG_INF, L = 0.f;
+#pragma unroll
+        for (u32 j = 0; j < KP; j++) M = fmaxf(M, ml[j].x);
+        if constexpr (MANY)
+            for (u32 s = lane + 64 * KP; s < ns; s += 64) M = fmaxf(M, pair(s).x);
+        M = group_max<64>(M);
+        const float mu = (M == NEG_INF) ? 0.f : M;
+        auto weigh = [&](u32 s, float2 x) __attribute__((always_inline)) {
+            const float w = fast_exp2(x.x - mu);
+            s_w[wave * ns + s] = w;
+            L = fmaf(w, x.y, L);
         };
-        float2 ml0 = make_float2(NEG_INF, 0.f);
-        if (wave < ncol) ml0 = pair(wave, lane);
-        if (part < P) load_batch(part);
-        float *const s_w = (float *)s_buf;
-        for (u32 hh = wave; hh < ncol; hh += NT / 64) {
-            float2 ml = hh == wave ? ml0 : pair(hh, lane);
-            float M = ml.x;
-            for (u32 s = lane + 64; s < ns; s += 64) M = fmaxf(M, pair(hh, s).x);
-            M = group_max<64>(M);
-            const float mu = (M == NEG_INF) ? 0.f : M;
-            float L = 0.f;
-            for (u32 s = lane; s < ns; s += 64) {
-                if (s != lane) ml = pair(hh, s);
-                const float w = fast_exp2(ml.x - mu);
-                s_w[hh * ns + s] = w;
-                L = fmaf(w, ml.y, L);
-            }
-            L = group_sum<64>(L);
-            if (lane == 0) s_inv[hh] = 1.0f / L;
-        }
-        __syncthreads();
-        if (part < P) {
-            for (u32 s0 = part; s0 < ns; s0 += K * P) {
-                if (s0 != part) load_batch(s0);
 #pragma unroll
-                for (u32 k = 0; k < K; k++) {
-                    const u32 s = s0 + k * P;
-                    if (s < ns) {
-                        const float w = s_w[h * ns + s];
-                        O.x = fmaf(w, __uint_as_float(a[k][0]), O.x);
-                        O.y = fmaf(w, __uint_as_float(a[k][1]), O.y);
-                        O.z = fmaf(w, __uint_as_float(a[k][2]), O.z);
-                        O.w = fmaf(w, __uint_as_float(a[k][3]), O.w);
-                    }
-                }
-            }
-            if (part) s_o[tid] = O;
-        }
-        __syncthreads();
-        if (part == 0) {
-            for (u32 q = 1; q < P; q++) {
-                const float4 t = s_o[tid + q * COLS];
-                O.x += t.x; O.y += t.y; O.z += t.z; O.w += t.w;
-            }
-            inv = s_inv[h];
-        }
-    } else {
-        if (part == 0) load_batch(0);
-        for (u32 i = tid; i < ncol * ns; i += NT) {
-            const u32x2v_t ml = __builtin_amdgcn_raw_buffer_load_b64(rml, i * 8, 0, TL_SC1);
-            s_buf[i] = make_float2(__uint_as_float(ml[0]), __uint_as_float(ml[1]));
-        }
-        __asm__ volatile("s_waitcnt vmcnt(0)" ::: "memory");
-        __syncthreads();
-        if (part == 0) {
-            float M = NEG_INF, L = 0.f;
-            const float2 *mlh = s_buf + h * ns;
-            for (u32 s0 = 0; s0 < ns; s0 += K) {
-                if (s0) load_batch(s0);
-                float2 ml[K];
-                float bm = NEG_INF;
+        for (u32 j = 0; j < KP; j++)
+            if (lane + 64 * j < ns) weigh(lane + 64 * j, ml[j]);
+        if constexpr (MANY)
+            for (u32 s = lane + 64 * KP; s < ns; s += 64) weigh(s, pair(s));
+        L = group_sum<64>(L);
+        if (lane == 0) s_inv[wave] = 1.0f / L;
+    }
+    __syncthreads();
+    if (part < P) {
+        for (u32 s0 = part; s0 < ns; s0 += K * P) {
+            if (s0 != part) load_batch(s0);
 #pragma unroll
-                for (u32 k = 0; k < K; k++) {
-                    const u32 s = s0 + k;
-                    ml[k] = mlh[min(s, ns - 1)];
-                    if (s >= ns) ml[k] = make_float2(NEG_INF, 0.f);   /* past the last split */
-                    bm = fmaxf(bm, ml[k].x);
-                }
-                const float nm = fmaxf(M, bm);
-                const float mu = (nm == NEG_INF) ? 0.f : nm;
-                const float sc = fast_exp2(M - mu);
-                L *= sc;
-                O.x *= sc; O.y *= sc; O.z *= sc; O.w *= sc;
-                M = nm;
-#pragma unroll
-                for (u32 k = 0; k < K; k++) {
-                    const float w = fast_exp2(ml[k].x - mu);
-                    L = fmaf(w, ml[k].y, L);
+            for (u32 k = 0; k < K; k++) {
+                const u32 s = s0 + k * P;
+                if (s < ns) {
+                    const float w = s_w[h * ns + s];
                     O.x = fmaf(w, __uint_as_float(a[k][0]), O.x);
                     O.y = fmaf(w, __uint_as_float(a[k][1]), O.y);
                     O.z = fmaf(w, __uint_as_float(a[k][2]), O.z);
                     O.w = fmaf(w, __uint_as_float(a[k][3]), O.w);
                 }
             }
-            inv = 1.0f / L;
         }
+        if (part) s_o[tid] = O;
     }
-    if (part == 0)
+    __syncthreads();
+    if (part == 0) {
+        for (u32 q = 1; q < P; q++) {
+            const float4 t = s_o[tid + q * COLS];
+            O.x += t.x; O.y += t.y; O.z += t.z; O.w += t.w;
+        }
+        const float inv = s_inv[h];
         *(float4 *)&sq.dst[(u64)(r + h / gh) * p.q_stride + (u64)(kvh * gh + h % gh) * D + d] =
             make_float4(O.x * inv, O.y * inv, O.z * inv, O.w * inv);
+    }
+}
+
+/* COLS_MAX: most columns of an instance's groups */
+template <int D, int NT, int COLS_MAX>
+TL_DEV void split_merge_regs(const DecParams &p, u32 pb, const float2 *ml_g, u32 ns, u32 kvh,
+                             u32 r, u32 gh, u32 ncol, const DecSeq &sq, float2 *s_buf) {
+    constexpr int TPC = pow2_floor(NT / COLS_MAX);
+    const bool few = ncol * (D / 4) <= NT / 4;
+    if (__builtin_expect(ns > 64, 0)) {
+        if (few && TPC < 16 && (TPC != 2 || ns > 96))
+            split_merge_shares<D, NT, true>(p, pb, ml_g, ns, kvh, r, gh, ncol, sq, s_buf);
+        else
+            split_merge_fold<D, NT, TPC>(p, pb, ml_g, ns, kvh, r, gh, ncol, sq, s_buf);
+    } else if (few && ns > 2 * TL_MERGE_TRIP) {
+        split_merge_shares<D, NT, false>(p, pb, ml_g, ns, kvh, r, gh, ncol, sq, s_buf);
+    } else if (D == 64 && TPC == 2 && ns > TL_MERGE_TRIP) {
+        split_merge_fold<D, NT, TPC>(p, pb, ml_g, ns, kvh, r, gh, ncol, sq, s_buf);
+    } else {
+        split_merge_fold<D, NT, 1>(p, pb, ml_g, ns, kvh, r, gh, ncol, sq, s_buf);
+    }
 }
 
 /* Bounded waits of the in-launch split merge (polls of device-coherent
@@ -1744,7 +1814,7 @@ __device__ __attribute__((always_inline)) inline void decode_ring_body(const Dec
     if (!closer) return;
     /* (m, l) pairs of the partials: cg * n_split <= 2048 (ring memory) */
     static_assert(CGT * D / 4 <= NT, "a merging thread per column");
-    split_merge_regs<D, NT>(p, pb, ml_g, n_split, kvh, r, G, cg, sq, (float2 *)&s_ring[0][0]);
+    split_merge_regs<D, NT, CGT * D / 4>(p, pb, ml_g, n_split, kvh, r, G, cg, sq, (float2 *)&s_ring[0][0]);
 }
 
 /* The kernel: slot indices staged as u32, at most TL_DEC_MAX_CHUNK keys per

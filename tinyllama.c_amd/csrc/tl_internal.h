@@ -91,12 +91,16 @@ struct DecParams {
 #define TL_MERGE_MAX_SPLIT_DIST 64
 /* A group's last workgroup merges all of it, unless there is much for one CU to
  * read and enough splits to share it: then every split merges a slice, at one
- * more round trip each.  A slice takes its workgroup's 8 waves one float4 each,
- * so 16 or fewer per split are two rounds.  us per launch, last workgroup /
- * slices, at head_dim 128 (columns = rows x heads of a group): 16 columns x 32
- * splits (256 KB of partials) 16.8 / 16.3, 8 x 32 (128 KB) 15.0 / 14.7, 7 x 64
- * 16.9 / 15.0; but 4 x 32 (64 KB) 28.1 / 28.3, 14 x 21 (147 KB, three rounds)
- * 14.6 / 15.3, 7 x 16 10.1 / 11.3. */
+ * more round trip each.  Few columns (output float4s = rows x heads x head_dim
+ * / 4): from the count on that takes the last workgroup a second trip, 8 rows
+ * of each of threads / columns shares; more columns: from 72 KB of partials.  A
+ * slice takes its workgroup's 8 waves one float4 each, so 16 or fewer per split
+ * are two rounds.  us per launch, last workgroup / slices, at head_dim 128
+ * (rows x heads of a group): 16 x 32 splits (256 KB) 16.8 / 16.3, 8 x 32 (128
+ * KB) 15.0 / 14.7, 7 x 64 16.9 / 15.0; but 4 x 32 (64 KB, one trip) 28.1 /
+ * 28.3, 14 x 21 (147 KB, three rounds) 14.6 / 15.3, 7 x 16 10.1 / 11.3; at 64, 7
+ * x 40 (two trips) 8.7 / 7.8, 5 x 56 8.5 / 7.8, 7 x 32 (one) 7.9 / 7.8. */
+#define TL_MERGE_TRIP 8
 #define TL_MERGE_MIN_SPLIT_DIST 24
 #define TL_MERGE_MIN_BYTES_DIST (72u << 10)
 #define TL_MERGE_SLICE_MAX 16
