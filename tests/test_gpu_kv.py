@@ -589,6 +589,30 @@ def test_few_heads_and_very_many_keys_take_the_prefill_kernel(T):
     assert times[0] < 1.5 * times[1], times
 
 
+def test_sixteen_rows_stay_on_the_decode_kernel(T):
+    """16 rows are appended by the decode launch itself: the plan takes it where
+    it is the faster one (measured 14.2 / 19.4 us; the bound is between)."""
+    import tlkv
+    n_head, n_kv, hd, pos, n = 32, 8, 64, 12500, 16
+    g = T.Generator(device="cuda")
+    g.manual_seed(n)
+    L = tlkv.Layer(pos + n, n_kv, hd)
+    q, k, v = (T.randn((n, h * hd), generator=g, device="cuda") for h in (n_head, n_kv, n_kv))
+    a = tlkv.attn_args(q, k, v, T.zeros_like(q), None, pos, n, n_head, hd, n_kv, 0, O.scale_of(hd))
+    times = {0: [], 2: []}
+    for _ in range(8):
+        for kernel, t in times.items():     # the plan's, the prefill kernel
+            with tlkv.tuning(tlkv.TUNE_NO_PREFILL, kernel):
+                e0, e1 = (T.cuda.Event(enable_timing=True) for _ in range(2))
+                e0.record()
+                for _ in range(20):
+                    tlkv.check(tlkv.lib().tl_attn(L.desc, a, tlkv.stream_handle()))
+                e1.record()
+                T.cuda.synchronize()
+                t.append(e0.elapsed_time(e1))
+    assert min(times[0]) < 0.88 * min(times[2]), times
+
+
 # windows that reach past the first key hide nothing, up to "no limit" as the
 # largest number and the last ones whose sum with a position passes 2^32
 @pytest.mark.parametrize("window", [2 ** 32 - 1, 2 ** 32 - 600, 2 ** 31, 900])

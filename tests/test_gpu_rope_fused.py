@@ -46,6 +46,8 @@ CASES = [
     (8, 4, 64, 200, 40, 32, 0, 1e4),         # prefill, head_dim 64, partial NORM
     (32, 8, 64, 700, 1, 64, 0, 5e5),         # decode, head_dim 64 (config 1 shape)
     (8, 4, 256, 600, 64, 256, 1, 1e6),       # prefill, head_dim 256, NEOX (config 5 global)
+    (32, 8, 128, 7000, 16, 128, 0, 5e5),     # 16 rows: decode kernel where 17 take prefill,
+    (32, 8, 128, 9900, 16, 128, 1, 1e6),     # and past its own line
 ]
 
 

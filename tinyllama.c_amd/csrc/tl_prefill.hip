@@ -223,7 +223,13 @@ bool tl_prefill_supported(const LayerView &L, const tl_attn_args *a) {
  * 26.2 / 27.8, 87K 42.0 / 34.8; Q8_0, 64 rows 14K 21.1 / 23.3, 16K 21.6 / 23.7;
  * 1/1/64, 64 rows 103K 19.3 / 32.5, 17 rows 221K 26.8 / 41.1 — but 349K 246 /
  * 50: past TL_DEC_FOLD_MAX_KEYS the chunks of a slot table make more splits than
- * a folded group merges (16 columns x 128), and each row reads the keys again. */
+ * a folded group merges (16 columns x 128), and each row reads the keys again.
+ * Up to TL_DEC_MAX_NEW rows the decode launch appends them itself and the line
+ * lies higher at head_dim <= 128: 16 rows, decode / prefill kernel, 32/8/128 over
+ * 6.1K keys 17.5 / 19.7, 10.4K 22.3 / 23.2, 13.4K 26.0 / 25.1; 28/4/128 7K 18.0 /
+ * 20.3, 11.9K 24.2 / 23.3; 32/8/64 12.2K 14.2 / 19.4, 20.8K 20.2 / 23.4; Q8_0, 32/8/128
+ * 3.8K 18.0 / 21.3, 6.5K 23.2 / 25.5, 28/4/128 7.4K 24.8 / 24.6; 8/4/256 6.1K 22.9 /
+ * 22.4. */
 #define TL_DEC_FOLD_MAX_KEYS (TL_DEC_MAX_CHUNK * 2048u / 16u)
 static u64 prefill_min_work(const LayerView &L) {
     const bool wide = L.head_dim == 256;
@@ -236,8 +242,10 @@ bool tl_use_prefill(const LayerView &L, const tl_attn_args *a) {
     if (tl_tune(TL_TUNE_NO_PREFILL) == 2) return true;
     const u64 keys = (u64)a->pos + a->n;
     const u64 vis = (a->window && keys > a->window) ? a->window : keys;
+    u64 most = prefill_min_work(L);
+    if (a->n <= TL_DEC_MAX_NEW && L.head_dim <= 128) most += most / 5 * 3;
     return a->n > TL_DEC_FOLD_MAX_ROWS || vis > TL_DEC_FOLD_MAX_KEYS ||
-           (u64)a->n * vis * a->n_head * L.head_dim > prefill_min_work(L);
+           (u64)a->n * vis * a->n_head * L.head_dim > most;
 }
 
 /* workgroups of W tasks per kv-head; GN = tasks of a 32-row block */
