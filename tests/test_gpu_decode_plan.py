@@ -98,15 +98,16 @@ def test_batch_of_unequal_sessions(T, case, slots):
 # n_head, n_kv, hd, keys, keys per split: split counts at the edges of a trip
 # (8), of two trips (16, 17) and of a wave (64, 65), where the group's last
 # workgroup merges; and both sides of the count from which every split merges a
-# slice: at least 24, 72 KB of partials and an output float4 in 16 per split, so
-# 24 for 7 or 8 heads at head_dim 128, 36 for 4, 32 for 8 heads at 256, 36 for
-# 2, and never (72, 288: more than the 64 it is limited to) for 4 or 1 at 64
+# slice: at least 24, an output float4 in 16 per split, and with at most 128
+# float4s a second trip of the last workgroup, else 72 KB of partials: 24 for 7
+# or 8 heads at head_dim 128, 33 for 4, 32 for 8 heads at 256, 33 for 2, and
+# never (65, 257: more than the 64 it is limited to) for 4 or 1 at 64
 MERGES = [(32, 8, 128, 64 * n, 64) for n in (2, 8, 9, 16, 17, 23, 24, 32)] + [
     (7, 1, 128, 64 * 64, 64), (7, 1, 128, 64 * 65, 64), (8, 1, 256, 64 * 40, 64),
     (1, 1, 64, 128 * 33, 128), (4, 1, 128, 64 * 200, 64), (8, 4, 256, 32 * 39, 32)] + [
     (7, 1, 128, 64 * 23, 64), (7, 1, 128, 64 * 24, 64), (16, 2, 128, 64 * 24, 64),
-    (16, 4, 128, 64 * 35, 64), (16, 4, 128, 64 * 36, 64), (8, 1, 256, 64 * 31, 64),
-    (8, 1, 256, 64 * 32, 64), (4, 2, 256, 32 * 35, 32), (4, 2, 256, 32 * 36, 32),
+    (16, 4, 128, 64 * 32, 64), (16, 4, 128, 64 * 33, 64), (8, 1, 256, 64 * 31, 64),
+    (8, 1, 256, 64 * 32, 64), (4, 2, 256, 32 * 32, 32), (4, 2, 256, 32 * 33, 32),
     (8, 2, 64, 128 * 64, 128)]
 
 

@@ -950,8 +950,8 @@ def test_decode_split_merge_fallback(T, shape):
     arrive merges all of them; with one poll some do and some do not.  The
     outputs equal the default run's bit for bit (every slice is merged by
     the same code from the same partials, whoever runs it).  32 splits of 4
-    heads (the first shape) have too few bytes for slices: their last split
-    merges and nothing waits; the others have 64 splits of 7 and of 4 heads and
+    heads (the first shape) are too few for slices: their last split merges in
+    one trip and nothing waits; the others have 64 splits of 7 and of 4 heads and
     40 of 8 heads at head_dim 256."""
     import tlkv
     n_head, n_kv, hd, cap, pos = shape
