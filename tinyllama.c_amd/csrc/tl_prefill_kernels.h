@@ -143,8 +143,13 @@ __global__ __attribute__((amdgpu_flat_work_group_size(64 * W, 64 * W), amdgpu_wa
     const u32 wq0 = p.pos + qb * 32;
     const u32 wq1 = p.pos + min(qb * 32 + 31, p.n - 1);
     /* first key the wave's first row sees (compared, never window + position:
-     * a window may be as large as 2^32 - 1) */
+     * a window may be as large as 2^32 - 1), and the tiles the wave works on,
+     * tb - tile0 < tile_n: from the first that reaches that key to its last row's (none
+     * without a task).  One scalar compare per tile: the three conditions apart,
+     * one of them in a vector register, took 512 rows over 32K keys 2 us */
     const u32 wk0 = (p.window && wq0 + 1 > p.window) ? wq0 + 1 - p.window : 0u;
+    const u32 tile0 = __builtin_amdgcn_readfirstlane(wk0 > BN - 1 ? wk0 - (BN - 1) : 0u);
+    const u32 tile_n = __builtin_amdgcn_readfirstlane(busy ? wq1 + 1 - tile0 : 0u);
 
     /* key range of the workgroup's rows, then of this split */
     const u32 wg_last = p.pos + min(((t0 + W - 1) / GN + 1) * 32, p.n);
@@ -366,7 +371,7 @@ __global__ __attribute__((amdgpu_flat_work_group_size(64 * W, 64 * W), amdgpu_wa
         const uint4 *sk = s_k[buf];
         const _Float16 *sv_t = s_v[buf];
         /* tiles past the wave's last row or before its first window: nothing */
-        if (busy && tb <= wq1 && tb + BN > wk0) {
+        if (tb - tile0 < tile_n) {
 
         /* S^T - mu = K . Q^T + bias per 32-key block (the accumulators start
          * at -mu, this row's running reference): lane holds keys
